@@ -141,6 +141,12 @@ hipError_t launch_generic_kernel(const AttnParams& p, dim3 grid, bool windowed, 
 hipError_t launch_rows_kernel(const AttnParams& p, dim3 grid, bool windowed, bool q_f16,
                               hipStream_t stream);
 int32_t rows_block_tokens(int32_t group);
+// The wide-block kernel (attn_wide.hip; paged cell caches, head size 64, 128
+// or 256, windowed / non-causal at 128 only, one split only at 64 and 256)
+// and the query tokens of one of its blocks.
+hipError_t launch_wide_kernel(const AttnParams& p, dim3 grid, bool windowed, bool q_f16,
+                              int head_size, hipStream_t stream);
+int32_t wide_block_tokens(int32_t head_size, int32_t group);
 hipError_t launch_combine_kernel(const CombineParams& c, hipStream_t stream);
 hipError_t launch_fill_unused_splits(const CombineParams& c, hipStream_t stream);
 

@@ -78,6 +78,16 @@ void set_cell_geometry(const PthAttnArgs& a, AttnParams& p) {
   p.cell_head = static_cast<uint32_t>(sh);
 }
 
+// Launches with more than this many query rows per request and KV head on
+// average run on the wide-block kernel: more rows than one 64-row tile holds.
+// Measured (unit kernels -> wide, 4 and 32 requests of 500 to 4,000 keys): at
+// 68 rows D = 128 36 -> 36 and 150 -> 132 us, D = 64 58 -> 28 and 319 -> 95,
+// D = 256 37 -> 35 and 113 -> 93; at 384 rows 80 -> 60 and 432 -> 273, 155 ->
+// 47 and 946 -> 208, 69 -> 61 and 351 -> 276. One launch of a 2,048-token
+// chunk and 60 decodes of up to 32k keys: 2,016 -> 1,865, 5,597 -> 1,270 and
+// 2,534 -> 1,762 us.
+constexpr int64_t kWideMinRows = 64;
+
 }  // namespace
 
 int32_t resident_workgroups() {
@@ -274,8 +284,22 @@ int32_t launch_attention(const PthAttnArgs& a, int32_t loader,
   // Head sizes 64 and 256: the register-load kernel (any block size).
   const bool d128 = a.head_size == 128;
   const bool row_blocks = d128 && a.num_splits == 1 && paged16 && rows >= 64;
+  // Prefill launches that the row-block kernel does not take: with split
+  // partials (their combine reads the split counts the kernel records, so
+  // only on that path), and at the other head sizes.
+  const bool wide = paged16 && !row_blocks && rows > 2 * kRowsPerWave &&
+                    (a.num_splits > 1 ? !fill_unused_splits : !d128) &&
+                    static_cast<int64_t>(a.num_tokens) * group >
+                        static_cast<int64_t>(a.num_reqs) * kWideMinRows;
   hipError_t err;
-  if (!d128) {
+  if (wide) {
+    p.blk_tok = wide_block_tokens(a.head_size, group);
+    const int64_t blocks =
+        (static_cast<int64_t>(a.num_tokens) / p.blk_tok + a.num_reqs) * a.num_kv_heads;
+    PA_REQUIRE(blocks < 0x7fffffff, "the block table exceeds 2^31 - 1 blocks");
+    const dim3 grid(static_cast<unsigned>(a.num_splits > 1 || blocks > wg_fill ? wg_fill : blocks));
+    err = launch_wide_kernel(p, grid, windowed, a.q_dtype == PTH_ATTN_F16, a.head_size, stream);
+  } else if (!d128) {
     const dim3 grid(static_cast<unsigned>(wg));
     err = launch_generic_kernel(p, grid, false, a.q_dtype == PTH_ATTN_F16, a.head_size, stream);
   } else if (row_blocks) {
