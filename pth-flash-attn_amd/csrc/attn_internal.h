@@ -69,9 +69,10 @@ struct AttnParams {
   int32_t blk_tok;
   int32_t num_kv_heads;
   float scale_log2;  // softmax_scale * log2(e)
-  // The page-row kernel applies (attn_staged.hip): the cell view is vLLM's
-  // NHD cell of 8 KV heads (264-byte cells, 2112-byte slot rows), pages of a
-  // multiple of 16 keys, and a work-group's 8 waves are the 8 KV heads.
+  // The page-row kernels apply (attn_staged.hip at D = 128, attn_paged64.hip at
+  // D = 64): the cell view is vLLM's NHD cell of 8 KV heads (cells of 2 D + 8
+  // bytes, slot rows of 8 cells), pages of a multiple of 16 keys, and a
+  // work-group's 8 waves are the 8 KV heads.
   int32_t page_rows;
 };
 
@@ -136,6 +137,8 @@ hipError_t launch_staged_kernel(const AttnParams& p, dim3 grid, bool windowed, b
                                 hipStream_t stream);
 hipError_t launch_generic_kernel(const AttnParams& p, dim3 grid, bool windowed, bool q_f16,
                                  int head_size, hipStream_t stream);
+// The D = 64 unit kernels on paged cell caches (attn_paged64.hip).
+hipError_t launch_paged64_kernel(const AttnParams& p, dim3 grid, bool q_f16, hipStream_t stream);
 // The row-block kernel (num_splits == 1, paged cell caches) and the query
 // tokens of one of its blocks for GQA group `group`.
 hipError_t launch_rows_kernel(const AttnParams& p, dim3 grid, bool windowed, bool q_f16,

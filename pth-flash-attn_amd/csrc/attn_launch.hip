@@ -252,11 +252,12 @@ int32_t launch_attention(const PthAttnArgs& a, int32_t loader,
   p.num_kv_heads = a.num_kv_heads;
   p.scale_log2 = a.softmax_scale * kLog2e;
   p.page_rows = 0;
-  if (p.cell && a.head_size == 128 && a.num_kv_heads == 8 && n_rg == 1 &&
-      a.block_size % 16 == 0 && p.cell_head == 264 && p.cell_slot == 8 * 264) {
-    bool inside = true;  // every stream of head h lies in bytes [264 h, 264 h + 264) of the row
+  const uint32_t cell = static_cast<uint32_t>(2 * a.head_size + 8);
+  if (p.cell && a.head_size <= 128 && a.num_kv_heads == 8 && n_rg == 1 &&
+      a.block_size % 16 == 0 && p.cell_head == cell && p.cell_slot == 8 * cell) {
+    bool inside = true;  // every stream of head h lies in bytes [cell h, cell h + cell) of the row
     for (int i = 0; i < 4; ++i)
-      inside = inside && p.cell_off[i] + (i < 2 ? 128u : 4u) <= 264u;
+      inside = inside && p.cell_off[i] + (i < 2 ? static_cast<uint32_t>(a.head_size) : 4u) <= cell;
     p.page_rows = inside ? 1 : 0;
   }
 
@@ -299,6 +300,9 @@ int32_t launch_attention(const PthAttnArgs& a, int32_t loader,
     PA_REQUIRE(blocks < 0x7fffffff, "the block table exceeds 2^31 - 1 blocks");
     const dim3 grid(static_cast<unsigned>(a.num_splits > 1 || blocks > wg_fill ? wg_fill : blocks));
     err = launch_wide_kernel(p, grid, windowed, a.q_dtype == PTH_ATTN_F16, a.head_size, stream);
+  } else if (a.head_size == 64 && paged16) {
+    const dim3 grid(static_cast<unsigned>(wg));
+    err = launch_paged64_kernel(p, grid, a.q_dtype == PTH_ATTN_F16, stream);
   } else if (!d128) {
     const dim3 grid(static_cast<unsigned>(wg));
     err = launch_generic_kernel(p, grid, false, a.q_dtype == PTH_ATTN_F16, a.head_size, stream);
