@@ -78,15 +78,24 @@ void set_cell_geometry(const PthAttnArgs& a, AttnParams& p) {
   p.cell_head = static_cast<uint32_t>(sh);
 }
 
-// Launches with more than this many query rows per request and KV head on
-// average run on the wide-block kernel: more rows than one 64-row tile holds.
-// Measured (unit kernels -> wide, 4 and 32 requests of 500 to 4,000 keys): at
-// 68 rows D = 128 36 -> 36 and 150 -> 132 us, D = 64 58 -> 28 and 319 -> 95,
-// D = 256 37 -> 35 and 113 -> 93; at 384 rows 80 -> 60 and 432 -> 273, 155 ->
-// 47 and 946 -> 208, 69 -> 61 and 351 -> 276. One launch of a 2,048-token
-// chunk and 60 decodes of up to 32k keys: 2,016 -> 1,865, 5,597 -> 1,270 and
-// 2,534 -> 1,762 us.
-constexpr int64_t kWideMinRows = 64;
+// Query rows per request and KV head, on average, from which a launch runs on
+// the wide-block kernel: below, its few blocks of long steps leave the chip
+// idle. The keys of a request are not known here, so the line lies where the
+// shortest prefill (no prefix) is as fast on either side; a prefix only adds
+// to the gain. Measured with split partials, unit kernels -> wide, without a
+// prefix and with one of 3,000 keys: D = 128, 8 query heads per KV head, 160
+// tokens (1,280 rows) 33 -> 34 and 147 -> 82 us over 4 requests, 330 tokens 60
+// -> 55 and 288 -> 148; 4 query heads, 83 tokens 22 -> 27, 700 tokens 119 -> 91
+// and 599 -> 281. D = 64, 4 query heads, 160 tokens 31 -> 33 and 99 -> 71, 700
+// tokens 95 -> 85 and 375 -> 214. D = 256 (half the rows a block), 330 tokens 51
+// -> 56 and 213 -> 171, 700 tokens 94 -> 88 and 416 -> 307; one request of 700
+// 46 -> 49. On a single split there are blocks enough: D = 64, 64 requests of 24
+// tokens 30 -> 32 us, with 300 keys before them 76 -> 46; D = 256, 64 requests
+// of 83 tokens 42 -> 47 and 118 -> 101, 16 of 330 96 -> 79 and 168 -> 135.
+constexpr int64_t wide_min_rows(int32_t head_size, int32_t num_splits) {
+  if (num_splits == 1) return head_size == 256 ? 384 : 64;
+  return head_size == 256 ? 3072 : 1280;
+}
 
 }  // namespace
 
@@ -282,7 +291,9 @@ int32_t launch_attention(const PthAttnArgs& a, int32_t loader,
   // Row tiles of 64 rows (the planner's prefill and wide-verify plans) on a
   // single split: the row-block kernel, whose 8 waves share each key chunk
   // (one work-group per CU, never more than there are blocks).
-  // Head sizes 64 and 256: the register-load kernel (any block size).
+  // Head size 64 on paged cells: its page-row and staged kernels. Other caches
+  // and head size 256: the register-load kernel (any block size) and, in its
+  // launcher, the direct-to-LDS kernel.
   const bool d128 = a.head_size == 128;
   const bool row_blocks = d128 && a.num_splits == 1 && paged16 && rows >= 64;
   // Prefill launches that the row-block kernel does not take: with split
@@ -290,8 +301,8 @@ int32_t launch_attention(const PthAttnArgs& a, int32_t loader,
   // only on that path), and at the other head sizes.
   const bool wide = paged16 && !row_blocks && rows > 2 * kRowsPerWave &&
                     (a.num_splits > 1 ? !fill_unused_splits : !d128) &&
-                    static_cast<int64_t>(a.num_tokens) * group >
-                        static_cast<int64_t>(a.num_reqs) * kWideMinRows;
+                    static_cast<int64_t>(a.num_tokens) * group >=
+                        a.num_reqs * wide_min_rows(a.head_size, a.num_splits);
   hipError_t err;
   if (wide) {
     p.blk_tok = wide_block_tokens(a.head_size, group);

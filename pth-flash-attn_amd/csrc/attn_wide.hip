@@ -26,8 +26,9 @@
 // is a power of two and the pending P of the previous step can be rescaled
 // without rounding. The largest p times the largest V scale of a step stays
 // below 2^15 (VScaleLimit): the V scales' binary exponent is part of the
-// growth threshold, no extra arithmetic. An fp16 query takes K in fp16 (one
-// product instead of the unit kernels' two).
+// growth threshold, no extra arithmetic unless they spread over more than
+// 2^8. An fp16 query takes K in fp16 (one product instead of the unit kernels'
+// two).
 //
 // Pipeline. Step k multiplies K(k) with Q, then runs softmax(k) while the
 // matrix unit works on P(k - 1) V(k - 1), which is independent of it: a step
@@ -405,13 +406,19 @@ struct WideState {
 
 constexpr float kNeverSeen = -3.402823466e38f;  // thr of a row without a visible key yet
 
-// The V scales seen so far are below 2^exp; p vs < 2^15 holds while
+// The V scales seen so far are in [lo, 2^exp); p vs < 2^15 holds while
 // score - m <= 15 - exp. A row whose max grows past that takes its new m so
-// that the max sits at 7 - exp.
+// that the max sits at 7 - exp. Once the scales of a segment spread over more
+// than 2^8, a row's large ones may be masked or without weight for it, and P
+// placed by them would lose its small ones: from then on (spread) the row's
+// largest p vs takes the place of the largest score, and exp is 0.
 struct VScaleLimit {
   int exp = -60;
   float lim = 0x1p-60f;
+  float lo = 0x1p126f;
+  bool spread = false;
 };
+constexpr float kVScaleSpread = 0x1p8f;
 
 // O *= alpha. With one wave per SIMD, O lives in accumulation registers, which
 // the vector unit cannot use: said in the operand constraints, since
@@ -711,15 +718,27 @@ void attn_fwd_wide(const AttnParams p) {
               if (key < L.lo || key > L.hi) t[tt][e] = kNegInf;
             }
         }
-        const float vsl = *reinterpret_cast<const float*>(vs_src + sb);
-        if (__ballot(vsl >= vl.lim) != 0) {  // a V scale beyond the bound: raise it
-          float vmax = vsl;
+        const float vsl = fabsf(*reinterpret_cast<const float*>(vs_src + sb));
+        // A V scale beyond the bounds (a key outside the segment has 0): they move.
+        if (__ballot(vsl >= vl.lim || (vsl < vl.lo && vsl > 0.0f)) != 0) {
+          float vmax = vsl, vmin = vsl > 0.0f ? vsl : vl.lo;
 #pragma unroll
-          for (int dd = 1; dd < 64; dd <<= 1) vmax = fmaxf(vmax, __shfl_xor(vmax, dd));
+          for (int dd = 1; dd < 64; dd <<= 1) {
+            vmax = fmaxf(vmax, __shfl_xor(vmax, dd));
+            vmin = fminf(vmin, __shfl_xor(vmin, dd));
+          }
           int e = static_cast<int>((__builtin_bit_cast(uint32_t, vmax) >> 23) & 0xff) - 126;
           e = e > 126 ? 126 : e;
+          e = e > vl.exp ? e : vl.exp;
           vl.exp = sgpr(e);
           vl.lim = __builtin_ldexpf(1.0f, vl.exp);
+          vl.lo = __builtin_bit_cast(float, sgpr(__builtin_bit_cast(int, fminf(vmin, vl.lo))));
+          if (vl.lim > vl.lo * (2.0f * kVScaleSpread)) {
+            vl.spread = true;
+            vl.exp = 0;
+            vl.lim = __builtin_inff();
+            vl.lo = 0.0f;
+          }
           st.thr = st.thr == kNeverSeen ? st.thr : static_cast<float>(15 - vl.exp);
         }
         float mx;
@@ -734,6 +753,18 @@ void attn_fwd_wide(const AttnParams p) {
           mx = max_raw(max3_raw(a[0], a[1], a[2]), a[3]);
           if constexpr (W::kTiles == 2)
             mx = max3_raw(mx, max_raw(a[4], a[5]), max_raw(a[6], a[7]));
+        }
+        if (vl.spread) {  // the largest p vs (a vs below 2^-60 as 2^-60, which bounds p)
+          mx = kNegInf;
+#pragma unroll
+          for (int tt = 0; tt < W::kTiles; ++tt)
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {
+              const f32x4 vs = *reinterpret_cast<const f32x4*>(s_src + sb + 4 * W::kStep + 128 * tt + 32 * b);
+#pragma unroll
+              for (int e = 0; e < 4; ++e)
+                mx = fmaxf(mx, t[tt][4 * b + e] + __builtin_amdgcn_logf(fmaxf(fabsf(vs[e]), 0x1p-60f)));
+            }
         }
         if (__ballot(mx > st.thr) != 0) {
           float shift;

@@ -20,42 +20,52 @@ from test_attn_gpu import check_case, run_capi, run_op
 pytestmark = pytest.mark.gpu
 
 
+def min_rows(D: int, S: int) -> int:
+    """Mean query rows per request from which the launcher takes the kernel."""
+    if S == 1:
+        return 384 if D == 256 else 64
+    return 3072 if D == 256 else 1280
+
+
 def wide(c: Case, S: int) -> bool:
     """The launcher's rule (attn_launch.hip)."""
     plan = c.plan()
     bq = tile_tokens(plan.wm, c.G, max(c.q_lens))
     return (c.block_size % 16 == 0 and bq * c.G > 32 and (S > 1 or c.D != 128)
-            and c.T * c.G > 64 * len(c.q_lens))
+            and c.T * c.G >= min_rows(c.D, S) * len(c.q_lens))
 
 
 def cases():
     for D in (64, 128, 256):
         blk = 128 if D == 256 else 256  # rows of a block
         step = 32 if D == 256 else 64  # keys of a step
+        m = min_rows(D, 2) // 4  # tokens of a request at four query heads per KV head
         heads = {"Hq": 8, "Hkv": 2, "D": D}
         # One block less, just, and more than full; keys at the step's edges.
-        for i, (rows, keys) in enumerate([(blk - 4, step), (blk, step + 1), (blk + 4, 2 * step - 1),
-                                          (3 * blk, 16 * step + 17)]):
-            q = rows // 4
-            yield Case(f"wide-d{D}-rows{rows}", q_lens=[q], seq_lens=[max(q, keys)], seed=400 + i,
-                       **heads)
-        yield Case(f"wide-d{D}-ragged", q_lens=[37, 0, 130, 1, 66, 40], seq_lens=[37, 9, 1500, 700, 67, 3000],
-                   seed=410, **heads)
-        yield Case(f"wide-d{D}-fp16q-hnd", q_lens=[100, 33], seq_lens=[900, 47], layout="HND",
+        for i, (rows, keys) in enumerate([(blk - 4, 0), (blk, 1), (blk + 4, step - 1), (3 * blk, 17)]):
+            q = m + rows // 4
+            yield Case(f"wide-d{D}-rows{rows}", q_lens=[q], seq_lens=[-(-q // step) * step + step + keys],
+                       seed=400 + i, **heads)
+        yield Case(f"wide-d{D}-first", q_lens=[m + 3], seq_lens=[m + 3], seed=409, **heads)
+        yield Case(f"wide-d{D}-ragged", q_lens=[m + 37, 0, 4 * m + 130, 1, m + 66, 40],
+                   seq_lens=[m + 37, 9, 4 * m + 1500, 700, m + 67, 3000], seed=410, **heads)
+        yield Case(f"wide-d{D}-fp16q-hnd", q_lens=[2 * m, 33], seq_lens=[2 * m + 800, 47], layout="HND",
                    q_dtype=torch.float16, seed=411, **heads)
-        yield Case(f"wide-d{D}-bs48", q_lens=[90, 50], seq_lens=[500, 1999], block_size=48, seed=412,
-                   Hq=12, Hkv=2, D=D)
-        yield Case(f"wide-d{D}-bs528-pad", q_lens=[70, 41], seq_lens=[1200, 300], block_size=528,
-                   pad_tokens=3, pad_page_bytes=72, seed=413, **heads)
-        yield Case(f"wide-d{D}-g64", q_lens=[5, 3], seq_lens=[333, 90], Hq=64, Hkv=1, D=D, seed=414)
-        yield Case(f"wide-d{D}-g1", q_lens=[300, 70], seq_lens=[300, 2000], Hq=3, Hkv=3, D=D, seed=415)
-        yield Case(f"wide-d{D}-many", q_lens=[20 + i % 9 for i in range(70)],
-                   seq_lens=[40 + 13 * i for i in range(70)], seed=416, **heads)
+        yield Case(f"wide-d{D}-bs48", q_lens=[m + 90, m], seq_lens=[m + 500, m + 1999], block_size=48,
+                   seed=412, Hq=12, Hkv=2, D=D)
+        yield Case(f"wide-d{D}-bs528-pad", q_lens=[m + 70, m + 41], seq_lens=[m + 1200, m + 300],
+                   block_size=528, pad_tokens=3, pad_page_bytes=72, seed=413, **heads)
+        yield Case(f"wide-d{D}-g64", q_lens=[m // 16 + 5, m // 16 + 3], seq_lens=[333, 90], Hq=64,
+                   Hkv=1, D=D, seed=414)
+        yield Case(f"wide-d{D}-g1", q_lens=[4 * m + 300, 4 * m + 70], seq_lens=[4 * m + 300, 4 * m + 500],
+                   Hq=2, Hkv=2, D=D, seed=415)
+        yield Case(f"wide-d{D}-many", q_lens=[m // 16 + i % 9 for i in range(70)],
+                   seq_lens=[m // 16 + 9 + 3 * i for i in range(70)], seed=416, Hq=64, Hkv=1, D=D)
     heads = {"Hq": 8, "Hkv": 2}
-    yield Case("wide-window", q_lens=[200, 40], seq_lens=[900, 3000], window=64, seed=420, **heads)
-    yield Case("wide-window-odd", q_lens=[131, 33], seq_lens=[2000, 800], window=333, seed=421, **heads)
-    yield Case("wide-noncausal", q_lens=[100, 30], seq_lens=[400, 50], causal=False, seed=422, **heads)
-    yield Case("wide-window-noncausal", q_lens=[80, 30], seq_lens=[2000, 300], window=100,
+    yield Case("wide-window", q_lens=[500, 400], seq_lens=[1200, 3000], window=64, seed=420, **heads)
+    yield Case("wide-window-odd", q_lens=[531, 133], seq_lens=[2000, 800], window=333, seed=421, **heads)
+    yield Case("wide-noncausal", q_lens=[600, 130], seq_lens=[900, 150], causal=False, seed=422, **heads)
+    yield Case("wide-window-noncausal", q_lens=[480, 330], seq_lens=[2000, 400], window=100,
                causal=False, seed=423, **heads)
 
 
@@ -72,7 +82,7 @@ def test_wide(case, S):
 def test_wide_op_and_repeats(D):
     """The op's launch (attention + combine) at the planner's split count, equal
     bit for bit over repeats."""
-    c = Case(f"wide-op-d{D}", q_lens=[150, 70], seq_lens=[2000, 333], Hq=8, Hkv=2, D=D, seed=430)
+    c = Case(f"wide-op-d{D}", q_lens=[1000, 600], seq_lens=[2000, 633], Hq=8, Hkv=2, D=D, seed=430)
     assert c.plan().num_splits > 1 and wide(c, c.plan().num_splits)
     b = materialize(c, "cuda")
     first = run_op(b)
@@ -83,13 +93,15 @@ def test_wide_op_and_repeats(D):
 
 
 @pytest.mark.parametrize("D", [64, 128, 256])
-@pytest.mark.parametrize("big", [2.0 ** 12, 2.0 ** 40])
+@pytest.mark.parametrize("big", [2.0 ** 3, 2.0 ** 6, 2.0 ** 12, 2.0 ** 40])
 def test_wide_large_v_scales(D, big):
     """V scales far beyond fp16's range that grow mid-stream: the growth
     threshold follows their exponent, so P V stays in range and rows that
-    grow rescale what they hold. Checked relative to each row's largest
+    grow rescale what they hold; once they spread too far the row's largest
+    p vs takes over, so the large scales of keys that are masked for a row, or
+    weigh nothing in it, cost the small ones no bits. Checked relative to each row's largest
     output: every step is fp32 or 22 bits, so 1e-5 leaves a decade."""
-    c = Case(f"wide-bigv-d{D}", q_lens=[96, 70], seq_lens=[300, 620], D=D, seed=440)
+    c = Case(f"wide-bigv-d{D}", q_lens=[800, 770], seq_lens=[800, 990], D=D, Hq=8, Hkv=2, seed=440)
     assert wide(c, 3)
     b = materialize(c, "cuda")
     ch, bt = b.cache, b.cache.block_table.cpu()
