@@ -11,7 +11,8 @@
 // or uninitialised memory) never enters an arithmetic operation; the sums run
 // in the fixed order s = 0..S-1, so the result is deterministic.
 //
-// Few rows with many splits (shared_rows): up to 512 splits, a work-group of
+// Few rows of few requests with many splits (shared_rows, chosen by the
+// launcher): up to 512 splits, a work-group of
 // 16 waves per (token, head) row and 32 of its columns (wave w merges split
 // block w, wave 0 merges the 16 results in a fixed order); beyond 512, one
 // work-group per row (wave w merges the 16-split blocks w, w + 16, ...).

@@ -78,6 +78,17 @@ void set_cell_geometry(const PthAttnArgs& a, AttnParams& p) {
   p.cell_head = static_cast<uint32_t>(sh);
 }
 
+// Requests up to which a launch's combine shares a row among the waves of a
+// work-group. The partition gives R requests about work-groups / R splits a
+// row, far below the launch's bound when R is large, and the sharing kernels'
+// loads of slots that hold no split then cost more than they hide: they read
+// the whole workspace. Measured, decode with its combine, one wave per row ->
+// shared (16q / 4kv heads, D = 128, 512 splits): 3 requests of 8k keys 26 -> 19
+// us, 6 26 -> 25, 8 27 -> 28, 12 30 -> 36, 24 42 -> 77; 24 of 700 keys 17 -> 33;
+// 4 of 300 to 32k 36 -> 27, 8 39 -> 38, 16 51 -> 75. D = 64 and 256 and 32 query
+// heads cross at 6 to 8 as well. Without the request lengths every split counts.
+constexpr int32_t kSharedCombineReqs = 8;
+
 // Query rows per request and KV head, on average, from which a launch runs on
 // the wide-block kernel: below, its few blocks of long steps leave the chip
 // idle. The keys of a request are not known here, so the line lies where the
@@ -405,7 +416,8 @@ int32_t launch_combine(const PthAttnCombineArgs& c, hipStream_t stream,
   p.head_size = c.head_size;
   if (split_source != nullptr) stream_fields(*split_source, p);
   const int64_t rows = static_cast<int64_t>(c.num_tokens) * c.num_q_heads;
-  p.shared_rows = c.num_splits > 64 && rows < 4 * static_cast<int64_t>(resident_workgroups());
+  p.shared_rows = c.num_splits > 64 &&
+                  (split_source == nullptr || c.num_reqs <= kSharedCombineReqs) && rows < 4 * static_cast<int64_t>(resident_workgroups());
   const hipError_t err = launch_combine_kernel(p, stream);
   if (err != hipSuccess) {
     return fail(PTH_ATTN_ECUDA, std::string("combine launch: ") + hipGetErrorString(err));
