@@ -50,6 +50,7 @@
 //   one softmax part forced after each product               206 us     314 us
 //   waves 4-7 half a step behind waves 0-3                  (spills)    347 us
 // D = 256 (12q / 2kv, 2,048 tokens at 4,099): 390 -> 267 us; with the ring 288.
+// The lower bound on the V scales and its branch cost 1, 2 and 3% of these.
 
 #include "attn_device.h"
 
