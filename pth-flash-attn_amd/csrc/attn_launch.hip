@@ -86,8 +86,12 @@ void set_cell_geometry(const PthAttnArgs& a, AttnParams& p) {
 // shared (16q / 4kv heads, D = 128, 512 splits): 3 requests of 8k keys 26 -> 19
 // us, 6 26 -> 25, 8 27 -> 28, 12 30 -> 36, 24 42 -> 77; 24 of 700 keys 17 -> 33;
 // 4 of 300 to 32k 36 -> 27, 8 39 -> 38, 16 51 -> 75. D = 64 and 256 and 32 query
-// heads cross at 6 to 8 as well. Without the request lengths every split counts.
-constexpr int32_t kSharedCombineReqs = 8;
+// heads cross at 6 to 8 as well. One request of 100k keys among short ones has
+// hundreds of splits, and one wave reads them in 32 round trips: 9 requests 63
+// -> 37, 16 61 -> 40, 31 63 -> 52 (32q / 8kv 66 -> 71, D = 256 84 -> 96). The
+// line is where even lengths gain more than this loses. Without the request
+// lengths every split counts.
+constexpr int32_t kSharedCombineReqs = 16;
 
 // Query rows per request and KV head, on average, from which a launch runs on
 // the wide-block kernel: below, its few blocks of long steps leave the chip

@@ -15,7 +15,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("D", [64, 128, 256])
-@pytest.mark.parametrize("R", [8, 9, 31])
+@pytest.mark.parametrize("R", [16, 17, 31])
 @pytest.mark.parametrize("long", [200, 30000])
 def test_combine_choice(D, R, long):
     c = Case(f"combine-d{D}-r{R}-{long}", q_lens=[1] * R, seq_lens=[40 + 7 * i for i in range(R - 1)] + [long],
