@@ -5,7 +5,7 @@
 // A work-group takes a block of 32 query rows per wave (256 rows at D = 64
 // and 128, 128 rows at D = 256) of one request and one KV head, and all its
 // waves share one stream of keys: each step loads 8 keys per wave, converts
-// them once (K to the query's 16-bit type, V to fp16, both exact for int8)
+// them once (K to the query's 16-bit type, V to bf16, both exact for int8)
 // and every wave multiplies its rows with all of them. The unit kernels, which
 // these launches ran on before, pass over the keys once per 16 rows and
 // convert them each time.
@@ -20,15 +20,12 @@
 // both reads over the LDS banks (b128 reads 2.3 ns each with eight waves
 // against 26.8 without, transposing reads 1.7 against 3.4).
 //
-// Numerics. As the unit kernels of attn_fwd.hip, except: P is an fp16
-// hi + lo pair (22 significant bits; the unit kernels' bf16 pair has 16), and
-// the reference max of a row is a whole number, so that every rescale factor
-// is a power of two and the pending P of the previous step can be rescaled
-// without rounding. The largest p times the largest V scale of a step stays
-// below 2^15 (VScaleLimit): the V scales' binary exponent is part of the
-// growth threshold, no extra arithmetic unless they spread over more than
-// 2^8. An fp16 query takes K in fp16 (one product instead of the unit kernels'
-// two).
+// Numerics. As the unit kernels of attn_fwd.hip: P is a bf16 hi + lo pair (16
+// significant bits at any size), a row's reference max moves when a score
+// exceeds it by more than kRescaleSlack. Here it is a whole number, so that
+// every rescale factor is a power of two and the pending P of the previous
+// step is rescaled without rounding. An fp16 query takes K in fp16 (one product
+// instead of the unit kernels' two).
 //
 // Pipeline. Step k multiplies K(k) with Q, then runs softmax(k) while the
 // matrix unit works on P(k - 1) V(k - 1), which is independent of it: a step
@@ -40,17 +37,21 @@
 // its 32 cycles (measured with independent fmas beside it), so per step and
 // wave at D = 128 the 48 products, ~330 vector instructions and 32 exp2 take
 // at least 2,220 cycles, two waves per SIMD 4,440; a step takes ~6,100, at
-// 1.84 GHz. Measured, with the same results (D = 128: 16q / 4kv, a chunk of
-// 2,011 tokens at 6,101 of a prefix, this kernel alone; D = 64: 32q / 8kv,
-// chunks of 1,108 and 1,389 tokens at 7,548 and 4,187, the whole call):
-//   unit kernels                                            510 us   2,124 us
-//   this                                                    195 us     303 us
+// 1.84 GHz. Measured, this kernel alone (D = 128: 16q / 4kv, a chunk of 2,011
+// tokens at 6,101 of a prefix, fp16; D = 64: 32q / 8kv, chunks of 1,108 and 1,389
+// tokens at 7,548 and 4,187; D = 256: 12q / 2kv, 2,048 tokens at 4,099):
+//                   D = 128    D = 64   D = 256
+//   unit kernels     460 us  2,091 us    375 us
+//   this             201       270       246
+// Tried on a version with P in fp16 (195 us; D = 64 303 us for the whole call):
 //   64 rows per wave, one wave per SIMD, half the LDS reads  206 us     348 us
 //   cache bytes direct to a ring in LDS, 2-4 steps ahead     202 us     314 us
 //   one softmax part forced after each product               206 us     314 us
 //   waves 4-7 half a step behind waves 0-3                  (spills)    347 us
-// D = 256 (12q / 2kv, 2,048 tokens at 4,099): 390 -> 267 us; with the ring 288.
-// The lower bound on the V scales and its branch cost 1, 2 and 3% of these.
+// P in fp16 has 22 bits near a row's largest p, but a floor: weights 2^18 and more
+// below the largest lost bits or vanished from the output while l counted them
+// (measured: up to a quarter of an element's sum of p |v|, 3e-3 of it on a long
+// context with one large V scale).
 
 #include "attn_device.h"
 
@@ -58,7 +59,7 @@ namespace pa {
 namespace {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef int16_t i16x4 __attribute__((ext_vector_type(4)));
 
@@ -344,7 +345,7 @@ __device__ __forceinline__ u32x2 i8x4_to_bf16(uint32_t w) {
 }
 
 // Converts word pair i of a step's bytes (the K words, then the V words) and
-// writes it row-major: K as the query's 16-bit type, V as fp16.
+// writes it row-major: K as the query's 16-bit type, V as bf16.
 template <int D, bool kF16Q>
 __device__ __forceinline__ void wide_stage_pair(const WideRaw<D>& r, int i, char* kdst,
                                                 char* vdst) {
@@ -352,8 +353,8 @@ __device__ __forceinline__ void wide_stage_pair(const WideRaw<D>& r, int i, char
   const bool is_v = i >= kHalf;
   const int w = 2 * (is_v ? i - kHalf : i);
   const uint32_t w0 = is_v ? r.v[w] : r.k[w], w1 = is_v ? r.v[w + 1] : r.k[w + 1];
-  const u32x2 a = is_v || kF16Q ? i8x4_to_f16(w0) : i8x4_to_bf16(w0);
-  const u32x2 b = is_v || kF16Q ? i8x4_to_f16(w1) : i8x4_to_bf16(w1);
+  const u32x2 a = kF16Q && !is_v ? i8x4_to_f16(w0) : i8x4_to_bf16(w0);
+  const u32x2 b = kF16Q && !is_v ? i8x4_to_f16(w1) : i8x4_to_bf16(w1);
   *reinterpret_cast<u32x4*>((is_v ? vdst : kdst) + 8 * w) = (u32x4){a[0], a[1], b[0], b[1]};
 }
 
@@ -377,20 +378,20 @@ __device__ __forceinline__ f32x16 wide_qk(const u32x4& k, const u32x4& q, f32x16
                                                    __builtin_bit_cast(bf16x8, q), c, 0, 0, 0);
 }
 
-// Column l % 32 of four consecutive keys of a row-major fp16 V (see above).
-__device__ __forceinline__ f16x4 v_column(const char* a) {
+// Column l % 32 of four consecutive keys of a row-major bf16 V (see above).
+__device__ __forceinline__ bf16x4 v_column(const char* a) {
   return __builtin_bit_cast(
-      f16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+      bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
                  (i16x4 __attribute__((address_space(3)))*)(const_cast<char*>(a))));
 }
 
 // V operand of output tile j and sub-product s: 32 columns of 16 keys, from
 // the V buffer whose lane address is `v`.
 template <int D>
-__device__ __forceinline__ f16x8 v_operand(const char* v, int s, int j) {
+__device__ __forceinline__ bf16x8 v_operand(const char* v, int s, int j) {
   constexpr int kVRow = WideDim<D>::kVRow;
-  const f16x4 x = v_column(v + (16 * s) * kVRow + 64 * j);
-  const f16x4 y = v_column(v + (16 * s + 8) * kVRow + 64 * j);
+  const bf16x4 x = v_column(v + (16 * s) * kVRow + 64 * j);
+  const bf16x4 y = v_column(v + (16 * s + 8) * kVRow + 64 * j);
   return __builtin_shufflevector(x, y, 0, 1, 2, 3, 4, 5, 6, 7);
 }
 
@@ -399,27 +400,11 @@ __device__ __forceinline__ f16x8 v_operand(const char* v, int s, int j) {
 template <int D>
 struct WideState {
   f32x16 o[WideDim<D>::kO];
-  f16x8 ph[WideDim<D>::kSub], pl[WideDim<D>::kSub];  // P of the previous step
+  bf16x8 ph[WideDim<D>::kSub], pl[WideDim<D>::kSub];  // P of the previous step
   float m;    // reference max (log2 units, a whole number); 0 before the first key
-  float thr;  // the row's m moves when a score minus m exceeds this
+  float thr;  // the row's m moves when a score minus m exceeds this (rescale_threshold)
   float l;
 };
-
-constexpr float kNeverSeen = -3.402823466e38f;  // thr of a row without a visible key yet
-
-// The V scales seen so far are in [lo, 2^exp); p vs < 2^15 holds while
-// score - m <= 15 - exp. A row whose max grows past that takes its new m so
-// that the max sits at 7 - exp. Once the scales of a segment spread over more
-// than 2^8, a row's large ones may be masked or without weight for it, and P
-// placed by them would lose its small ones: from then on (spread) the row's
-// largest p vs takes the place of the largest score, and exp is 0.
-struct VScaleLimit {
-  int exp = -60;
-  float lim = 0x1p-60f;
-  float lo = 0x1p126f;
-  bool spread = false;
-};
-constexpr float kVScaleSpread = 0x1p8f;
 
 // O *= alpha. With one wave per SIMD, O lives in accumulation registers, which
 // the vector unit cannot use: said in the operand constraints, since
@@ -452,25 +437,57 @@ __device__ __forceinline__ void wide_scale_o(WideState<D>& st, float alpha) {
   }
 }
 
+// P *= alpha, a power of two: exact.
+__device__ __forceinline__ bf16x8 scale_p(bf16x8 p, float alpha) {
+  const u32x4 w = __builtin_bit_cast(u32x4, p);
+  u32x4 r;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float a = __builtin_bit_cast(float, w[i] << 16) * alpha;
+    const float b = __builtin_bit_cast(float, w[i] & 0xffff0000u) * alpha;
+    r[i] = __builtin_bit_cast(uint32_t, pack_bf16(a, b));
+  }
+  return __builtin_bit_cast(bf16x8, r);
+}
+
 template <int D>
-__device__ __forceinline__ void wide_grow(WideState<D>& st, float lane_mx, int vexp,
-                                          float& shift) {
+__device__ __forceinline__ void wide_grow(WideState<D>& st, float lane_mx, float& shift) {
   const SwapPair sw = swap_halves(lane_mx);
   const float mx = max_raw(sw.a, sw.b);
   const bool grow = mx > st.thr;
-  shift = grow ? ceilf(mx - static_cast<float>(7 - vexp)) : 0.0f;
+  shift = grow ? ceilf(mx) : 0.0f;
   // A row's first visible key: nothing accumulated, any factor.
-  const float alpha = grow && st.thr != kNeverSeen ? __builtin_amdgcn_exp2f(-shift) : 1.0f;
-  const _Float16 a16 = static_cast<_Float16>(alpha);
+  const float alpha =
+      grow && st.thr == kRescaleSlack ? __builtin_amdgcn_exp2f(-shift) : 1.0f;
   st.l *= alpha;
   wide_scale_o(st, alpha);
 #pragma unroll
   for (int s = 0; s < WideDim<D>::kSub; ++s) {
-    st.ph[s] *= a16;
-    st.pl[s] *= a16;
+    st.ph[s] = scale_p(st.ph[s], alpha);
+    st.pl[s] = scale_p(st.pl[s], alpha);
   }
   st.m += shift;
-  st.thr = grow ? static_cast<float>(15 - vexp) : st.thr;
+  st.thr = grow ? kRescaleSlack : st.thr;
+}
+
+// Two P V weights -> bf16 hi + lo. x - hi is exact, and one instruction: a dot
+// product with a pair that picks the element. The pairs are kept in registers:
+// as a constant, {-1, 0} becomes the instruction's inline -1.0, whose bits are
+// those of the fp32 value, {0, -1}.
+struct Picks {
+  uint32_t first = 0x0000bf80u, second = 0xbf800000u;  // bf16 {-1, 0}, {0, -1}
+  __device__ __forceinline__ void keep() { asm volatile("" : "+s"(first), "+s"(second)); }
+};
+struct PPair {
+  bf16x2 hi, lo;
+};
+__device__ __forceinline__ PPair p_pair(const Picks& k, float x, float y) {
+  PPair r;
+  r.hi = pack_bf16(x, y);
+  r.lo = pack_bf16(
+      __builtin_amdgcn_fdot2_f32_bf16(r.hi, __builtin_bit_cast(bf16x2, k.first), x, false),
+      __builtin_amdgcn_fdot2_f32_bf16(r.hi, __builtin_bit_cast(bf16x2, k.second), y, false));
+  return r;
 }
 
 // O += P V of 16 keys: sub-product s of the step whose V rows are at `v`
@@ -478,15 +495,15 @@ __device__ __forceinline__ void wide_grow(WideState<D>& st, float lane_mx, int v
 template <int D>
 __device__ __forceinline__ void wide_pv(WideState<D>& st, const char* v, int s) {
   constexpr int kO = WideDim<D>::kO;
-  f16x8 a[kO];
+  bf16x8 a[kO];
 #pragma unroll
   for (int j = 0; j < kO; ++j) a[j] = v_operand<D>(v, s, j);
 #pragma unroll
   for (int j = 0; j < kO; ++j)
-    st.o[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[j], st.ph[s], st.o[j], 0, 0, 0);
+    st.o[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[j], st.ph[s], st.o[j], 0, 0, 0);
 #pragma unroll
   for (int j = 0; j < kO; ++j)
-    st.o[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[j], st.pl[s], st.o[j], 0, 0, 0);
+    st.o[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[j], st.pl[s], st.o[j], 0, 0, 0);
 }
 
 // Stores of a finished segment: out, or the split's partial.
@@ -587,8 +604,9 @@ void attn_fwd_wide(const AttnParams p) {
   const char* const v_src = lds + W::kVBase + (4 * h + ((lane & 15) >> 2)) * W::kVRow +
                             32 * ((lane >> 4) & 1) + 8 * (lane & 3);
   const char* const s_src = lds + W::kSBase + 16 * h;
-  const char* const vs_src = lds + W::kSBase + 4 * W::kStep + 4 * (lane & (W::kStep - 1));
 
+  Picks picks;
+  picks.keep();
   WideWalk<kWindow, kStream> walk;
   walk.init(p, lane);
   Segment g;
@@ -605,9 +623,9 @@ void attn_fwd_wide(const AttnParams p) {
 #pragma unroll
     for (int s = 0; s < W::kSub; ++s)
 #pragma unroll
-      for (int e = 0; e < 8; ++e) st.ph[s][e] = st.pl[s][e] = static_cast<_Float16>(0.0f);
+      for (int e = 0; e < 8; ++e) st.ph[s][e] = st.pl[s][e] = static_cast<__bf16>(0.0f);
     st.m = 0.0f;
-    st.thr = kNeverSeen;
+    st.thr = rescale_threshold(true);
     st.l = 0.0f;
 
     const int c0 = g.lo & ~15;
@@ -635,7 +653,6 @@ void attn_fwd_wide(const AttnParams p) {
               (lane & 7) * static_cast<uint32_t>(W::kLaneBytes);
       wo.s = (8u * (wave & 1) + (lane & 7)) * p.cell_slot + cell_head +
              ((lane & 8) ? p.cell_off[3] : p.cell_off[2]);
-      VScaleLimit vl;
       WideRaw<D> raw;
       wide_load<D>(p, pw, wo, key_group(p, c0, wave, last16), raw);
       __syncthreads();  // the previous segment's reads of the buffers are done
@@ -719,29 +736,6 @@ void attn_fwd_wide(const AttnParams p) {
               if (key < L.lo || key > L.hi) t[tt][e] = kNegInf;
             }
         }
-        const float vsl = fabsf(*reinterpret_cast<const float*>(vs_src + sb));
-        // A V scale beyond the bounds (a key outside the segment has 0): they move.
-        if (__ballot(vsl >= vl.lim || (vsl < vl.lo && vsl > 0.0f)) != 0) {
-          float vmax = vsl, vmin = vsl > 0.0f ? vsl : vl.lo;
-#pragma unroll
-          for (int dd = 1; dd < 64; dd <<= 1) {
-            vmax = fmaxf(vmax, __shfl_xor(vmax, dd));
-            vmin = fminf(vmin, __shfl_xor(vmin, dd));
-          }
-          int e = static_cast<int>((__builtin_bit_cast(uint32_t, vmax) >> 23) & 0xff) - 126;
-          e = e > 126 ? 126 : e;
-          e = e > vl.exp ? e : vl.exp;
-          vl.exp = sgpr(e);
-          vl.lim = __builtin_ldexpf(1.0f, vl.exp);
-          vl.lo = __builtin_bit_cast(float, sgpr(__builtin_bit_cast(int, fminf(vmin, vl.lo))));
-          if (vl.lim > vl.lo * (2.0f * kVScaleSpread)) {
-            vl.spread = true;
-            vl.exp = 0;
-            vl.lim = __builtin_inff();
-            vl.lo = 0.0f;
-          }
-          st.thr = st.thr == kNeverSeen ? st.thr : static_cast<float>(15 - vl.exp);
-        }
         float mx;
         {
           float a[4 * W::kTiles];
@@ -755,31 +749,22 @@ void attn_fwd_wide(const AttnParams p) {
           if constexpr (W::kTiles == 2)
             mx = max3_raw(mx, max_raw(a[4], a[5]), max_raw(a[6], a[7]));
         }
-        if (vl.spread) {  // the largest p vs (a vs below 2^-60 as 2^-60, which bounds p)
-          mx = kNegInf;
-#pragma unroll
-          for (int tt = 0; tt < W::kTiles; ++tt)
-#pragma unroll
-            for (int b = 0; b < 4; ++b) {
-              const f32x4 vs = *reinterpret_cast<const f32x4*>(s_src + sb + 4 * W::kStep + 128 * tt + 32 * b);
-#pragma unroll
-              for (int e = 0; e < 4; ++e)
-                mx = fmaxf(mx, t[tt][4 * b + e] + __builtin_amdgcn_logf(fmaxf(fabsf(vs[e]), 0x1p-60f)));
-            }
-        }
         if (__ballot(mx > st.thr) != 0) {
           float shift;
-          wide_grow<D>(st, mx, vl.exp, shift);
+          wide_grow<D>(st, mx, shift);
 #pragma unroll
           for (int tt = 0; tt < W::kTiles; ++tt)
 #pragma unroll
             for (int e = 0; e < 16; ++e) t[tt][e] -= shift;
         }
-        // softmax(k), 8 scores per lane at a time, beside P(k - 1) V(k - 1).
+        // softmax(k), 8 scores per lane at a time, beside P(k - 1) V(k - 1). The
+        // step's p are summed before l takes them: added to l one by one, a long
+        // tail of small p would be rounded to l's last place each time.
+        float l_step = 0.0f;
 #pragma unroll
         for (int s = 0; s < W::kSub; ++s) {
           wide_pv<D>(st, v_src + vprev, s);
-          f16x8 ph, pl;
+          bf16x8 ph, pl;
 #pragma unroll
           for (int b = 0; b < 2; ++b) {
             const f32x4 vs =
@@ -788,23 +773,22 @@ void attn_fwd_wide(const AttnParams p) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
               const float pe = __builtin_amdgcn_exp2f(t[s >> 1][8 * (s & 1) + 4 * b + e]);
-              st.l += pe;
+              l_step = s + b + e == 0 ? pe : l_step + pe;
               pv[e] = pe * vs[e];
             }
 #pragma unroll
             for (int e = 0; e < 4; e += 2) {
-              const auto hi2 = __builtin_amdgcn_cvt_pkrtz(pv[e], pv[e + 1]);
-              const auto lo2 = __builtin_amdgcn_cvt_pkrtz(pv[e] - static_cast<float>(hi2[0]),
-                                                          pv[e + 1] - static_cast<float>(hi2[1]));
-              ph[4 * b + e] = hi2[0];
-              ph[4 * b + e + 1] = hi2[1];
-              pl[4 * b + e] = lo2[0];
-              pl[4 * b + e + 1] = lo2[1];
+              const PPair pp = p_pair(picks, pv[e], pv[e + 1]);
+              ph[4 * b + e] = pp.hi[0];
+              ph[4 * b + e + 1] = pp.hi[1];
+              pl[4 * b + e] = pp.lo[0];
+              pl[4 * b + e + 1] = pp.lo[1];
             }
           }
           st.ph[s] = ph;
           st.pl[s] = pl;
         }
+        st.l += l_step;
         kb = kn;
         sb = sn;
         vprev = vb;

@@ -4,8 +4,7 @@ D = 64 and 256, at the edges of its blocks, steps and score tiles.
 
 The gates are those of the unit kernels (test_attn_gpu.check_case): the
 output within the parity tolerance beyond its storage rounding, and the
-fp32-output launch within 1e-4. P is an fp16 hi + lo pair (22 significant
-bits), so the arithmetic error is that of the fp32 sums.
+fp32-output launch within 1e-4 (P is a bf16 hi + lo pair, as there).
 """
 
 from __future__ import annotations
@@ -14,7 +13,9 @@ import numpy as np
 import pytest
 import torch
 
-from cases import Case, assert_parity, compare, materialize, oracle_of, tile_tokens
+from cases import (
+    Batch, Case, abs_v_batch, assert_parity, compare, materialize, oracle_of, tile_tokens,
+)
 from test_attn_gpu import check_case, run_capi, run_op
 
 pytestmark = pytest.mark.gpu
@@ -95,12 +96,11 @@ def test_wide_op_and_repeats(D):
 @pytest.mark.parametrize("D", [64, 128, 256])
 @pytest.mark.parametrize("big", [2.0 ** 3, 2.0 ** 6, 2.0 ** 12, 2.0 ** 40])
 def test_wide_large_v_scales(D, big):
-    """V scales far beyond fp16's range that grow mid-stream: the growth
-    threshold follows their exponent, so P V stays in range and rows that
-    grow rescale what they hold; once they spread too far the row's largest
-    p vs takes over, so the large scales of keys that are masked for a row, or
-    weigh nothing in it, cost the small ones no bits. Checked relative to each row's largest
-    output: every step is fp32 or 22 bits, so 1e-5 leaves a decade."""
+    """V scales that grow mid-stream by factors far beyond fp16's range, of keys
+    that some rows see, that are masked for others, or that weigh nothing in
+    them: the small ones lose no bits. Checked relative to each row's largest
+    output: a term lies within 2^-17 = 7.6e-6 of itself, and the errors of a
+    row's terms are as good as independent."""
     c = Case(f"wide-bigv-d{D}", q_lens=[800, 770], seq_lens=[800, 990], D=D, Hq=8, Hkv=2, seed=440)
     assert wide(c, 3)
     b = materialize(c, "cuda")
@@ -114,5 +114,77 @@ def test_wide_large_v_scales(D, big):
     o, r = out.cpu().numpy()[valid].astype(np.float64), ref_out[valid]
     assert np.isfinite(o).all()
     rel = np.abs(o - r) / np.abs(r).max(axis=-1, keepdims=True)
+    print(f"large V scales d{D} {big:g}: worst {rel.max():.3g}")
     assert rel.max() <= 1e-5, rel.max()
     assert np.abs(lse.cpu().numpy()[valid] - ref_lse[valid]).max() <= 1e-3
+
+
+# ------------------------------------------------- weights far below the largest
+# The kernel's numerics are those of the unit kernels: P is a hi + lo pair of 16
+# significant bits at any size, so a term p_i v_i of a row's sum is within
+# 2^-17 of itself, and the scores, exponentials and fp32 sums add less than as
+# much again: the oracle on |V| gives sum_i p_i |v_i| / l, and every output
+# element lies within 2^-16 of that.
+P_PAIR_UNIT = 2.0 ** -16
+KEYS = 4096
+
+
+def _sink(n, step, x, r):
+    """Key 0 is 2^x above the rest, its V scale r times theirs."""
+    score, vs = np.zeros(n), np.ones(n)
+    score[0], vs[0] = x, r
+    return score, vs
+
+
+def _jump(n, step, x, r):
+    """One step of equal keys, then one key 2^x above them, nothing after it."""
+    score, vs = np.full(n, -80.0), np.ones(n)
+    score[:step], score[step], vs[step] = 0.0, x, r
+    return score, vs
+
+
+def _tail(n, step, x, r):
+    """Key 0 over a long tail 2^x below it, and a key of no weight whose V scale
+    is 1 / r times theirs."""
+    score, vs = np.full(n, -x), np.ones(n)
+    score[0], score[1], vs[1] = 0.0, -80.0, 1.0 / r
+    return score, vs
+
+
+def _small_weight_case(D, S):
+    return Case(f"wide-small-d{D}", q_lens=[min_rows(D, 2) // 4 + 9], seq_lens=[KEYS], D=D, Hq=4, Hkv=1,
+                seed=450)
+
+
+def _places(b, r, n):
+    t = torch.arange(n, device="cuda")
+    return b.cache.block_table[r, t // b.case.block_size].long(), t % b.case.block_size
+
+
+@pytest.mark.parametrize("ratio", [1.0, 1 / 8, 1 / 100, 1 / 300])
+@pytest.mark.parametrize("x", [17.5, 22.6, 25.0, 30.0])
+@pytest.mark.parametrize("profile", [_sink, _jump, _tail], ids=lambda f: f.__name__[1:])
+@pytest.mark.parametrize("D,S", [(64, 1), (64, 2), (128, 2), (256, 1), (256, 2)])
+def test_wide_small_weights(D, S, profile, x, ratio):
+    c = _small_weight_case(D, S)
+    assert wide(c, S)
+    b = materialize(c, "cuda")
+    b.q.fill_(1.0)
+    score, vs = profile(KEYS, 32 if D == 256 else 64, x, ratio)
+    pages, slots = _places(b, 0, KEYS)
+    ch = b.cache
+    ch.k_cache[pages, slots] = 1  # score = sqrt(D) k_scale
+    ch.k_scale[pages, slots] = torch.tensor(score * np.log(2) / np.sqrt(D), dtype=torch.float32, device="cuda")[:, None]
+    ch.v_scale[pages, slots] = torch.tensor(0.01 * vs, dtype=torch.float32, device="cuda")[:, None]
+    torch.cuda.synchronize()
+    # All rows have one query: the oracle on the last token's, which sees every key.
+    last = Case(c.name, q_lens=[1], seq_lens=[KEYS], D=D, Hq=4, Hkv=1)
+    lb = Batch(last, ch, b.q[-1:], torch.tensor([0, 1], dtype=torch.int32, device="cuda"))
+    ref_out, ref_lse, _ = oracle_of(lb, threads=16)
+    abs_out, _, _ = oracle_of(abs_v_batch(lb), threads=16)
+    out, lse = run_capi(b, num_splits=S, out_dtype=torch.float32)
+    err = np.abs(out[-1:].cpu().numpy().astype(np.float64) - ref_out)
+    worst = float((err / abs_out).max())
+    print(f"d{D} S{S} {profile.__name__} x={x} ratio={ratio:.4f}: worst error / sum p|v| {worst:.3g}")
+    assert worst <= P_PAIR_UNIT, worst
+    assert np.abs(lse[-1:].cpu().numpy() - ref_lse).max() <= 1e-3
