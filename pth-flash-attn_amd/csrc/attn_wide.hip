@@ -25,7 +25,8 @@
 // exceeds it by more than kRescaleSlack. Here it is a whole number, so that
 // every rescale factor is a power of two and the pending P of the previous
 // step is rescaled without rounding. An fp16 query takes K in fp16 (one product
-// instead of the unit kernels' two).
+// instead of the unit kernels' two). A key whose p is 0, masked or more than
+// 2^126 below the row's largest, adds nothing whatever its V scale.
 //
 // Pipeline. Step k multiplies K(k) with Q, then runs softmax(k) while the
 // matrix unit works on P(k - 1) V(k - 1), which is independent of it: a step
@@ -470,6 +471,10 @@ __device__ __forceinline__ void wide_grow(WideState<D>& st, float lane_mx, float
   st.thr = grow ? kRescaleSlack : st.thr;
 }
 
+// v_mul_legacy_f32 (no builtin): a product in which 0 times anything is 0. The p
+// of a masked key is 0, and its V scale may be any bits, also infinite or NaN.
+extern "C" __device__ float mul_legacy(float a, float b) __asm("llvm.amdgcn.fmul.legacy");
+
 // Two P V weights -> bf16 hi + lo. x - hi is exact, and one instruction: a dot
 // product with a pair that picks the element. The pairs are kept in registers:
 // as a constant, {-1, 0} becomes the instruction's inline -1.0, whose bits are
@@ -774,7 +779,7 @@ void attn_fwd_wide(const AttnParams p) {
             for (int e = 0; e < 4; ++e) {
               const float pe = __builtin_amdgcn_exp2f(t[s >> 1][8 * (s & 1) + 4 * b + e]);
               l_step = s + b + e == 0 ? pe : l_step + pe;
-              pv[e] = pe * vs[e];
+              pv[e] = mul_legacy(pe, vs[e]);
             }
 #pragma unroll
             for (int e = 0; e < 4; e += 2) {

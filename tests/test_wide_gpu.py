@@ -188,3 +188,39 @@ def test_wide_small_weights(D, S, profile, x, ratio):
     print(f"d{D} S{S} {profile.__name__} x={x} ratio={ratio:.4f}: worst error / sum p|v| {worst:.3g}")
     assert worst <= P_PAIR_UNIT, worst
     assert np.abs(lse[-1:].cpu().numpy() - ref_lse).max() <= 1e-3
+
+
+# ------------------------------------------------------------- non-finite inputs
+def _sees(c, r, key):
+    """Rows (tokens of the batch) that see position `key` of request r."""
+    seen = np.zeros(c.T, bool)
+    t0, n, L = sum(c.q_lens[:r]), c.q_lens[r], c.seq_lens[r]
+    p = np.arange(L - n, L)
+    seen[t0:t0 + n] = (p >= key) & ((c.window == 0) | (key >= p - c.window + 1))
+    return torch.from_numpy(seen).cuda()
+
+
+@pytest.mark.parametrize("stream", ["k_scale", "v_scale"])
+@pytest.mark.parametrize("bad", [float("inf"), float("-inf"), float("nan")])
+@pytest.mark.parametrize("D,S,window", [(64, 1, 0), (64, 2, 0), (128, 2, 0), (128, 2, 150), (256, 1, 0),
+                                        (256, 3, 0)])
+def test_wide_non_finite_scale(D, S, window, bad, stream):
+    """A non-finite scale reaches the rows that see its key, and no other row of
+    the block; a V scale never reaches a row's LSE."""
+    m = min_rows(D, 2) // 4
+    c = Case(f"wide-nonfinite-d{D}", q_lens=[m + 70, m], seq_lens=[m + 300, m + 41], window=window, D=D,
+             Hq=8, Hkv=2, seed=460)
+    assert wide(c, S)
+    b = materialize(c, "cuda")
+    clean, clean_lse = run_capi(b, num_splits=S, out_dtype=torch.float32)
+    key = c.seq_lens[0] - c.q_lens[0] + 133  # within a block's tokens
+    pages, slots = _places(b, 0, c.seq_lens[0])
+    getattr(b.cache, stream)[pages[key], slots[key]] = bad
+    out, lse = run_capi(b, num_splits=S, out_dtype=torch.float32)
+    seen = _sees(c, 0, key)
+    assert 0 < int(seen.sum()) < c.q_lens[0]
+    assert torch.equal(out[~seen].view(torch.int32), clean[~seen].view(torch.int32))
+    assert torch.equal(lse[~seen].view(torch.int32), clean_lse[~seen].view(torch.int32))
+    if stream == "v_scale":
+        assert not torch.isfinite(out[seen]).any()
+        assert torch.equal(lse.view(torch.int32), clean_lse.view(torch.int32))
