@@ -379,6 +379,20 @@ __device__ __forceinline__ f32x16 wide_qk(const u32x4& k, const u32x4& q, f32x16
                                                    __builtin_bit_cast(bf16x8, q), c, 0, 0, 0);
 }
 
+// A row with a non-finite fp16 query element gets a NaN one, so that all its
+// scores are NaN, as in the unit kernels (their hi + lo pair of an infinity is
+// inf, NaN): an infinity alone would give keys with a negative byte there the
+// score -inf, and drop them.
+template <int N>
+__device__ __forceinline__ void query_non_finite(u32x4 (&q)[N]) {
+  uint32_t any = 0;  // bit 15 of a half: the sum of a half with an exponent of all ones
+#pragma unroll
+  for (int j = 0; j < N; ++j)
+#pragma unroll
+    for (int w = 0; w < 4; ++w) any |= (q[j][w] & 0x7fff7fffu) + 0x04000400u;
+  if (any & 0x80008000u) q[0][0] |= 0x7fff7fffu;
+}
+
 // Column l % 32 of four consecutive keys of a row-major bf16 V (see above).
 __device__ __forceinline__ bf16x4 v_column(const char* a) {
   return __builtin_bit_cast(
@@ -651,6 +665,7 @@ void attn_fwd_wide(const AttnParams p) {
           q[j] = *reinterpret_cast<const u32x4*>(qrow + 32 * j + 16 * h);
           if (!L.vrow) q[j] = (u32x4){0u, 0u, 0u, 0u};
         }
+        if constexpr (kF16Q) query_non_finite(q);
       }
       WideOffsets wo;
       const uint32_t cell_head = static_cast<uint32_t>(g.kvh) * p.cell_head;

@@ -224,3 +224,22 @@ def test_wide_non_finite_scale(D, S, window, bad, stream):
     if stream == "v_scale":
         assert not torch.isfinite(out[seen]).any()
         assert torch.equal(lse.view(torch.int32), clean_lse.view(torch.int32))
+
+
+@pytest.mark.parametrize("D,S", [(64, 1), (128, 2), (256, 1)])
+def test_wide_infinite_query(D, S):
+    """A row whose fp16 query holds an infinity is NaN whatever the sign of the
+    keys' bytes there, and no other row changes."""
+    m = min_rows(D, 2) // 4
+    c = Case(f"wide-infq-d{D}", q_lens=[m + 33], seq_lens=[m + 90], D=D, Hq=8, Hkv=2, q_dtype=torch.float16,
+             seed=470)
+    assert wide(c, S)
+    b = materialize(c, "cuda")
+    b.cache.k_cache[..., 5] = -7
+    clean, _ = run_capi(b, num_splits=S, out_dtype=torch.float32)
+    row, head = 101, 3
+    b.q[row, head, 5] = float("inf")
+    out, _ = run_capi(b, num_splits=S, out_dtype=torch.float32)
+    assert torch.isnan(out[row, head]).all()
+    out[row, head] = clean[row, head]
+    assert torch.equal(out.view(torch.int32), clean.view(torch.int32))
