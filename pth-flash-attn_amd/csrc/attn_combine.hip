@@ -16,7 +16,8 @@
 // 16 waves per (token, head) row and 32 of its columns (wave w merges split
 // block w, wave 0 merges the 16 results in a fixed order); beyond 512, one
 // work-group per row (wave w merges the 16-split blocks w, w + 16, ...).
-// Otherwise one wave per row.
+// Few rows of many requests (few_rows): a work-group of 4 waves per row, of which
+// one works unless the row has more than 64 splits. Otherwise one wave per row.
 // The kernels are latency-bound, so the loads are ordered by round: the
 // padding bound, the split-count marker and the wave's LSEs are issued
 // together (the LSEs before their count is known; slots past it are then
@@ -347,6 +348,38 @@ __device__ __forceinline__ void write_row(const CombineParams& c, int64_t tok, i
   }
 }
 
+// The results of kN waves in LDS, all read at once (one LDS round trip), then
+// merged in wave order.
+template <int NC, int kN>
+__device__ __forceinline__ void merge_parts(const float (&part_m)[kN], const float (&part_den)[kN],
+                                            const float (&part_num)[kN][NC][64], int lane, float& M,
+                                            float (&num)[NC], float& den) {
+  float pm[kN], pd[kN], pn[kN][NC];
+#pragma unroll
+  for (int w = 0; w < kN; ++w) {
+    pm[w] = part_m[w];
+    pd[w] = part_den[w];
+#pragma unroll
+    for (int i = 0; i < NC; ++i) pn[w][i] = part_num[w][i][lane];
+  }
+  M = kNegInf;
+#pragma unroll
+  for (int w = 0; w < kN; ++w) M = pm[w] > M ? pm[w] : M;
+#pragma unroll
+  for (int i = 0; i < NC; ++i) num[i] = 0.0f;
+  den = 0.0f;
+  if (!(M > kNegInf)) return;
+#pragma unroll
+  for (int w = 0; w < kN; ++w) {
+    if (pm[w] > kNegInf) {
+      const float a = __builtin_amdgcn_exp2f(pm[w] - M);
+#pragma unroll
+      for (int i = 0; i < NC; ++i) num[i] = fmaf(a, pn[w][i], num[i]);
+      den = fmaf(a, pd[w], den);
+    }
+  }
+}
+
 // One wave per (token, head) row, whatever its split count.
 template <int D>
 __global__ __launch_bounds__(256) void combine_splits(const CombineParams c) {
@@ -378,6 +411,131 @@ __global__ __launch_bounds__(256) void combine_splits(const CombineParams c) {
     merge_one_block<NC, 64, kSpec>(c, tok, head, S, 0, x_spec, ov_spec, lane, M, num, den);
   else
     merge_blocks<NC>(c, tok, head, S, 0, 1, lane, M, num, den);
+  write_row<NC>(c, tok, head, M, num, den, lane);
+}
+
+// Few rows of many requests (few_rows without shared_rows): most rows have few
+// splits, a long request's have hundreds. A work-group of kRowWaves waves per
+// row: a row whose splits fit one 64-split block is merged by the first wave, as
+// in combine_splits, and the others leave as soon as they know the count; the
+// splits of a longer row are cut into kRowWaves runs, one per wave, and wave 0
+// merges the results in a fixed order. One wave alone walks up to 512 splits
+// in 32 dependent rounds of loads; the sharing kernels read the slots of every
+// planned split of the short rows. Decode with its combine, 24 requests, one of
+// 100k keys among 500: one wave per row 61, sharing kernel 46, this 35 us (16q /
+// 4kv, D = 128; D = 256 74, 55, 38; D = 64 54, 44, 27); 24 of 700 keys 14, 33, 14;
+// 24 of 8k keys 41, 74, 41. With 8 waves the long rows take 1 to 4 us less and
+// 31 requests of 700 keys (32q / 8kv) 23.6 us against 22.5 (one wave 21.9);
+// with partial rows of 64 splits in flight it is between the two.
+constexpr int kRowWaves = 4;
+
+// Merge of splits [lo, hi): their maximum log2-LSE M and, relative to it, this
+// lane's NC numerator columns and the (wave-summed) denominator. The partial
+// rows of kB splits are in flight together; splits past hi read hi - 1 again and,
+// like those without weight, enter no sum.
+template <int NC>
+__device__ __forceinline__ void merge_run(const CombineParams& c, int64_t tok, int head, int lo,
+                                          int hi, int lane, float& M, float (&num)[NC],
+                                          float& den) {
+  constexpr int kB = NC == 4 ? 16 : 32;
+  const char* lse_row = c.ws_lse + tok * c.s_wl_tok + static_cast<int64_t>(head) * c.s_wl_head;
+  const char* o_row =
+      c.ws_o + tok * c.s_wo_tok + static_cast<int64_t>(head) * c.s_wo_head + 4 * NC * lane;
+  auto lse_at = [&](int s) {
+    return s < hi ? *reinterpret_cast<const float*>(lse_row + s * c.s_wl_split) : kNegInf;
+  };
+  float x = lse_at(lo + lane);
+  M = x > kNegInf ? x : kNegInf;  // NaN never wins
+  for (int s0 = lo + 64; s0 < hi; s0 += 64) {
+    const float y = lse_at(s0 + lane);
+    M = y > M ? y : M;
+  }
+  M = wave_max(M);
+#pragma unroll
+  for (int i = 0; i < NC; ++i) num[i] = 0.0f;
+  den = 0.0f;
+  if (!(M > kNegInf)) return;
+  float den_l = 0.0f;
+  for (int s0 = lo; s0 < hi; s0 += 64) {
+    const float w_l = x > kNegInf ? __builtin_amdgcn_exp2f(x - M) : 0.0f;
+    den_l += w_l;
+    x = lse_at(s0 + 64 + lane);
+    for (int e0 = 0; e0 < 64 && s0 + e0 < hi; e0 += kB) {
+      float ov[kB][NC];
+#pragma unroll
+      for (int k = 0; k < kB; ++k) {
+        const int s = s0 + e0 + k;
+        load_cols<NC>(o_row + (s < hi ? s : hi - 1) * c.s_wo_split, ov[k]);
+      }
+#pragma unroll
+      for (int k = 0; k < kB; ++k) {
+        const float w = __builtin_bit_cast(
+            float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, w_l), e0 + k));
+        if (w > 0.0f) {
+#pragma unroll
+          for (int i = 0; i < NC; ++i) num[i] = fmaf(w, ov[k][i], num[i]);
+        }
+      }
+    }
+  }
+  den = wave_sum(den_l);
+}
+
+template <int D>
+__global__ __launch_bounds__(kRowWaves * 64) void combine_rows(const CombineParams c) {
+  constexpr int NC = D / 64;
+  __shared__ float part_m[kRowWaves], part_den[kRowWaves];
+  __shared__ float part_num[kRowWaves][NC][64];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t row = blockIdx.x;
+  const int64_t tok = row / c.num_q_heads;
+  const int head = static_cast<int>(row - tok * c.num_q_heads);
+  if (tok >= c.num_tokens) return;  // uniform over the work-group
+  const int bound = ld_ro(c.qsl, c.num_reqs);
+  const uint32_t bits = marker_bits(c, tok, head);  // read on every path: the slot exists
+  float M, den;
+  float num[NC];
+  int S;
+  if (wave == 0) {  // one round of loads, as in combine_splits
+    const float x_spec = lse_slot<64>(c, tok, head, 0, lane);
+    constexpr int kSpec = 4;
+    float ov_spec[kSpec][NC];
+    spec_rows<NC, 64, kSpec>(c, tok, head, 0, lane, ov_spec);
+    asm volatile("" ::"s"(bits), "s"(bound) : "memory");
+    if (tok >= bound) return;  // padding row
+    S = c.seq_lens != nullptr ? splits_of_marker(c, bits) : c.num_splits;
+    if (c.seq_lens != nullptr && S == 1) return;  // written to out by the attention kernel
+    if (S <= 64) {
+      merge_one_block<NC, 64, kSpec>(c, tok, head, S, 0, x_spec, ov_spec, lane, M, num, den);
+      write_row<NC>(c, tok, head, M, num, den, lane);
+      return;
+    }
+  } else {
+    if (tok >= bound) return;
+    S = c.seq_lens != nullptr ? splits_of_marker(c, bits) : c.num_splits;
+    if (S <= 64) return;
+  }
+  // Every wave of the work-group is here, or none.
+  const int per = (S + kRowWaves - 1) / kRowWaves;
+  const int lo = wave * per, hi = lo + per < S ? lo + per : S;
+  if (lo < hi) {
+    merge_run<NC>(c, tok, head, lo, hi, lane, M, num, den);
+  } else {
+    M = kNegInf;
+    den = 0.0f;
+#pragma unroll
+    for (int i = 0; i < NC; ++i) num[i] = 0.0f;
+  }
+  if (lane == 0) {
+    part_m[wave] = M;
+    part_den[wave] = den;
+  }
+#pragma unroll
+  for (int i = 0; i < NC; ++i) part_num[wave][i][lane] = num[i];
+  __syncthreads();
+  if (wave != 0) return;
+  merge_parts<NC, kRowWaves>(part_m, part_den, part_num, lane, M, num, den);
   write_row<NC>(c, tok, head, M, num, den, lane);
 }
 
@@ -443,35 +601,8 @@ __global__ __launch_bounds__(kSharedWaves * 64) void combine_shared(const Combin
   for (int i = 0; i < NC; ++i) part_num[wave][i][lane] = num[i];
   __syncthreads();
   if (wave != 0) return;
-  // Every wave's result read at once (one LDS round trip), then merged in
-  // wave order.
-  float pm[kSharedWaves], pd[kSharedWaves], pn[kSharedWaves][NC];
-#pragma unroll
-  for (int w = 0; w < kSharedWaves; ++w) {
-    pm[w] = part_m[w];
-    pd[w] = part_den[w];
-#pragma unroll
-    for (int i = 0; i < NC; ++i) pn[w][i] = part_num[w][i][lane];
-  }
-  float Mg = kNegInf;
-#pragma unroll
-  for (int w = 0; w < kSharedWaves; ++w) Mg = pm[w] > Mg ? pm[w] : Mg;
-  float ng[NC];
-#pragma unroll
-  for (int i = 0; i < NC; ++i) ng[i] = 0.0f;
-  float dg = 0.0f;
-  if (Mg > kNegInf) {
-#pragma unroll
-    for (int w = 0; w < kSharedWaves; ++w) {
-      if (pm[w] > kNegInf) {
-        const float a = __builtin_amdgcn_exp2f(pm[w] - Mg);
-#pragma unroll
-        for (int i = 0; i < NC; ++i) ng[i] = fmaf(a, pn[w][i], ng[i]);
-        dg = fmaf(a, pd[w], dg);
-      }
-    }
-  }
-  write_row<NC>(c, tok, head, Mg, ng, dg, lane);
+  merge_parts<NC, kSharedWaves>(part_m, part_den, part_num, lane, M, num, den);
+  write_row<NC>(c, tok, head, M, num, den, lane);
 }
 
 // Few rows with up to 16 kBlk splits each, split by columns as well: a
@@ -614,6 +745,9 @@ void launch_combine_d(const CombineParams& c, int64_t rows, hipStream_t stream) 
   else if (c.shared_rows)
     hipLaunchKernelGGL((combine_shared<D, 16>), dim3(static_cast<unsigned>(rows)),
                        dim3(kSharedWaves * 64), 0, stream, c);
+  else if (c.few_rows)
+    hipLaunchKernelGGL(combine_rows<D>, dim3(static_cast<unsigned>(rows)), dim3(kRowWaves * 64), 0,
+                       stream, c);
   else
     hipLaunchKernelGGL(combine_splits<D>, dim3(static_cast<unsigned>((rows + kWaves - 1) / kWaves)),
                        dim3(kWaves * 64), 0, stream, c);

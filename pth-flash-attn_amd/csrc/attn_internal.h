@@ -106,10 +106,10 @@ struct CombineParams {
   int32_t num_wg;  // partition work-groups: attention work-groups x kGroupUnits / gu
   int32_t window;
   int32_t causal;
-  // A work-group per row (rows with many splits are merged by 4 waves)
-  // instead of a wave per row: set when the launch may have more than 64
-  // splits per row and has few rows.
-  int32_t shared_rows;
+  // few_rows: the launch may have more than 64 splits per row and has few rows.
+  // shared_rows: of these, the launches whose rows are each merged by the 16
+  // waves of a work-group; the others take one wave per row.
+  int32_t few_rows, shared_rows;
 };
 
 // Host launchers. They check their arguments, enqueue on `stream`, allocate

@@ -78,19 +78,18 @@ void set_cell_geometry(const PthAttnArgs& a, AttnParams& p) {
   p.cell_head = static_cast<uint32_t>(sh);
 }
 
-// Requests up to which a launch's combine shares a row among the waves of a
-// work-group. The partition gives R requests about work-groups / R splits a
-// row, far below the launch's bound when R is large, and the sharing kernels'
-// loads of slots that hold no split then cost more than they hide: they read
-// the whole workspace. Measured, decode with its combine, one wave per row ->
-// shared (16q / 4kv heads, D = 128, 512 splits): 3 requests of 8k keys 26 -> 19
-// us, 6 26 -> 25, 8 27 -> 28, 12 30 -> 36, 24 42 -> 77; 24 of 700 keys 17 -> 33;
-// 4 of 300 to 32k 36 -> 27, 8 39 -> 38, 16 51 -> 75. D = 64 and 256 and 32 query
-// heads cross at 6 to 8 as well. One request of 100k keys among short ones has
-// hundreds of splits, and one wave reads them in 32 round trips: 9 requests 63
-// -> 37, 16 61 -> 40, 31 63 -> 52 (32q / 8kv 66 -> 71, D = 256 84 -> 96). The
-// line is where even lengths gain more than this loses. Without the request
-// lengths every split counts.
+// Requests up to which the combine of a launch with few rows shares every row
+// among the 16 waves of a work-group, which load the slots of every planned split
+// at once. The partition gives R requests of like lengths about work-groups / R
+// splits a row, far below the plan's bound when R is large, and the loads of slots
+// that hold no split then cost more than they hide. Decode with its combine, 16q /
+// 4kv heads, D = 128, 512 splits planned, combine_rows -> shared: 17 requests of 8k
+// keys 34 -> 45 us, 24 41 -> 74, 24 of 700 keys 14 -> 33; one request of 100k
+// keys among 500: 17 requests 34 -> 41, 24 35 -> 46. Below the line one wave
+// per row -> shared: 3 of 8k keys 26 -> 19, 6 26 -> 25, 8 27 -> 28, 12 30 -> 36, 16
+// 51 -> 75 of 300 to 32k, and 16 with one of 100k 61 -> 38; combine_rows was not
+// measured there. Without the request lengths every split counts, so those
+// launches share at any R.
 constexpr int32_t kSharedCombineReqs = 16;
 
 // Query rows per request and KV head, on average, from which a launch runs on
@@ -420,8 +419,9 @@ int32_t launch_combine(const PthAttnCombineArgs& c, hipStream_t stream,
   p.head_size = c.head_size;
   if (split_source != nullptr) stream_fields(*split_source, p);
   const int64_t rows = static_cast<int64_t>(c.num_tokens) * c.num_q_heads;
-  p.shared_rows = c.num_splits > 64 &&
-                  (split_source == nullptr || c.num_reqs <= kSharedCombineReqs) && rows < 4 * static_cast<int64_t>(resident_workgroups());
+  p.few_rows = c.num_splits > 64 && rows < 4 * static_cast<int64_t>(resident_workgroups());
+  p.shared_rows =
+      p.few_rows && (split_source == nullptr || c.num_reqs <= kSharedCombineReqs);
   const hipError_t err = launch_combine_kernel(p, stream);
   if (err != hipSuccess) {
     return fail(PTH_ATTN_ECUDA, std::string("combine launch: ") + hipGetErrorString(err));

@@ -9,7 +9,7 @@ import pytest
 import torch
 
 from cases import Case, assert_parity, compare, materialize, oracle_of
-from test_attn_gpu import run_op
+from test_attn_gpu import run_capi, run_op
 
 pytestmark = pytest.mark.gpu
 
@@ -26,3 +26,20 @@ def test_combine_choice(D, R, long):
     ref, _, valid = oracle_of(b, threads=16)
     assert_parity(compare(out, None, ref, None, valid), name=c.name, strict=False)
     assert torch.equal(run_op(b).view(torch.int16), out.view(torch.int16))
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("chunks", [64, 65, 66, 127, 128, 129, 255, 256, 257, 262, 938])
+def test_long_row_among_short_ones(D, chunks):
+    """A row of exactly `chunks` live splits (one KV head: every chunk of a launch
+    this small is a split) beside rows of two, on the kernel that cuts a long
+    row into runs: one block, the last wave's run short or empty, runs of more
+    than a block; output and LSE."""
+    c = Case(f"combine-row-d{D}-{chunks}", q_lens=[1] * 17, seq_lens=[40] * 8 + [32 * chunks - 5] + [60] * 8,
+             Hq=4, Hkv=1, D=D, seed=620)
+    assert c.plan().num_splits > chunks
+    b = materialize(c, "cuda")
+    ref, ref_lse, valid = oracle_of(b, threads=16)
+    out, lse = run_capi(b, out_dtype=torch.float32)
+    res = compare(out, lse, ref, ref_lse, valid)
+    assert res["finite"] and res["max_abs"] <= 1e-4 and res["lse_max_abs"] <= 1e-3, res
