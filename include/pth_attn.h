@@ -204,6 +204,10 @@ int32_t pth_attn_has_cuda(void);
 /* Message of the calling thread's last failure ("" after a success).
  * Reference: attn_capi.h:87, attn_launch.h:46-56 */
 const char* pth_attn_last_error(void);
+/* Kernel of the calling thread's last attention launch (its name without
+ * template arguments; "" before the first). Tests assert with it that a case
+ * runs on the kernel it is about. No counterpart in the reference's ABI. */
+const char* pth_attn_last_kernel(void);
 
 /* Tiling of the kernel chosen for (head_size, bq, group): *n_tile = KV tokens
  * per tile (64), *sub_tile = KV tokens per softmax step (32), *wn = query-row

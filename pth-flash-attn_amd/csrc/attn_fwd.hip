@@ -168,6 +168,7 @@ constexpr int kShortWindow = 4096;
 template <bool W, bool St, bool F>
 hipError_t launch_paged(const AttnParams& p, dim3 grid, hipStream_t stream) {
   if (W && p.window > 0 && p.window <= kShortWindow) {
+    note_kernel("attn_fwd_paged_reg");
     hipLaunchKernelGGL((attn_fwd_paged_reg<W, St, F>), grid, dim3(kFwdWaves * 64), 0, stream, p);
     return hipGetLastError();
   }

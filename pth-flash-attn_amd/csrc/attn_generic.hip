@@ -342,6 +342,7 @@ bool use_paged256(const AttnParams& p) { return p.cell && p.bs_div.d % 16 == 0; 
 
 template <bool W, bool St, int D>
 hipError_t launch_d(const AttnParams& p, dim3 grid, bool q_f16, hipStream_t stream) {
+  note_kernel("attn_fwd_generic");
   if (q_f16)
     hipLaunchKernelGGL((attn_fwd_generic<W, St, true, D>), grid, dim3(kFwdWaves * 64), 0, stream,
                        p);
@@ -353,6 +354,7 @@ hipError_t launch_d(const AttnParams& p, dim3 grid, bool q_f16, hipStream_t stre
 
 template <bool St>
 hipError_t launch_paged256(const AttnParams& p, dim3 grid, bool q_f16, hipStream_t stream) {
+  note_kernel("attn_fwd_paged256");
   if (q_f16)
     hipLaunchKernelGGL((attn_fwd_paged256<St, true>), grid, dim3(kFwdWaves * 64), 0, stream, p);
   else

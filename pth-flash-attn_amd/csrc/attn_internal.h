@@ -156,6 +156,10 @@ hipError_t launch_fill_unused_splits(const CombineParams& c, hipStream_t stream)
 // The int8 cache writer (attn_writer.hip).
 int32_t launch_write_kv(const PthAttnWriteArgs& a, hipStream_t stream);
 
+// The kernel launchers record the name of the kernel they choose.
+void note_kernel(const char* name);
+const char* last_kernel();
+
 const char* last_error();
 int32_t fail(int32_t code, const std::string& msg);
 void clear_error();

@@ -19,6 +19,7 @@ namespace pa {
 namespace {
 
 thread_local std::string g_last_error;
+thread_local const char* g_last_kernel = "";
 
 constexpr float kLog2e = 1.44269504088896340736f;
 constexpr int64_t kVecAlign = 16;
@@ -128,6 +129,9 @@ int32_t resident_workgroups() {
   if (dev < kMaxDevices) cached[dev] = wgs;
   return wgs;
 }
+
+void note_kernel(const char* name) { g_last_kernel = name; }
+const char* last_kernel() { return g_last_kernel; }
 
 const char* last_error() { return g_last_error.c_str(); }
 int32_t fail(int32_t code, const std::string& msg) {
@@ -532,6 +536,7 @@ int32_t pth_attn_combine_args_bytes(void) {
 int32_t pth_attn_options_bytes(void) { return static_cast<int32_t>(sizeof(PthAttnOptions)); }
 int32_t pth_attn_has_cuda(void) { return 1; }
 const char* pth_attn_last_error(void) { return pa::last_error(); }
+const char* pth_attn_last_kernel(void) { return pa::last_kernel(); }
 
 int32_t pth_attn_tiling(int32_t head_size, int32_t bq, int32_t group,
                         int32_t* n_tile, int32_t* sub_tile, int32_t* wn) {

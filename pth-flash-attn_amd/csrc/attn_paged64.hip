@@ -375,6 +375,7 @@ void attn_fwd_staged64(const AttnParams p_arg) {
 
 hipError_t launch_paged64_kernel(const AttnParams& p, dim3 grid, bool q_f16, hipStream_t stream) {
   const bool st = p.num_splits > 1;
+  note_kernel(p.page_rows ? "attn_fwd_pagerows64" : "attn_fwd_staged64");
   const dim3 block(kFwdWaves * 64);
 #define PA_LAUNCH(K, St, F) hipLaunchKernelGGL((K<St, F>), grid, block, 0, stream, p)
   if (p.page_rows) {

@@ -1119,6 +1119,7 @@ void attn_fwd_rows(const AttnParams p) {
 
 hipError_t launch_rows_kernel(const AttnParams& p, dim3 grid, bool windowed, bool q_f16,
                               hipStream_t stream) {
+  note_kernel("attn_fwd_rows");
   const dim3 block(kRowWaves * 64);
   if (windowed) {
     if (q_f16) hipLaunchKernelGGL((attn_fwd_rows<true, true>), grid, block, 0, stream, p);

@@ -393,6 +393,7 @@ void attn_fwd_pagerows(const AttnParams p) {
 hipError_t launch_staged_kernel(const AttnParams& p, dim3 grid, bool windowed, bool q_f16,
                                 hipStream_t stream) {
   const bool st = p.num_splits > 1;
+  note_kernel(p.page_rows ? "attn_fwd_pagerows" : "attn_fwd_staged");
   if (p.page_rows) {
 #define PA_LAUNCH(W, St, F) \
   hipLaunchKernelGGL((attn_fwd_pagerows<W, St, F>), grid, dim3(kFwdWaves * 64), 0, stream, p)

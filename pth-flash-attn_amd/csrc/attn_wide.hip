@@ -843,6 +843,7 @@ int32_t wide_block_tokens(int32_t head_size, int32_t group) {
 hipError_t launch_wide_kernel(const AttnParams& p, dim3 grid, bool windowed, bool q_f16,
                               int head_size, hipStream_t stream) {
   const bool split = p.num_splits > 1;
+  note_kernel("attn_fwd_wide");
   if (head_size == 64)
     return split ? launch_wide<64, false, true>(p, grid, q_f16, stream)
                  : launch_wide<64, false, false>(p, grid, q_f16, stream);

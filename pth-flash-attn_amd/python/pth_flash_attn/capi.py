@@ -29,6 +29,7 @@ EXPORTED_SYMBOLS = (
     "pth_attn_options_bytes",
     "pth_attn_has_cuda",
     "pth_attn_last_error",
+    "pth_attn_last_kernel",
     "pth_attn_tiling",
     "pth_attn_attention",
     "pth_attn_attention_ex",
@@ -176,6 +177,8 @@ class AttnLib:
             getattr(lib, name).argtypes = []
         lib.pth_attn_last_error.restype = ctypes.c_char_p
         lib.pth_attn_last_error.argtypes = []
+        lib.pth_attn_last_kernel.restype = ctypes.c_char_p
+        lib.pth_attn_last_kernel.argtypes = []
         ip = ctypes.POINTER(i32)
         lib.pth_attn_tiling.restype = i32
         lib.pth_attn_tiling.argtypes = [i32, i32, i32, ip, ip, ip]
@@ -203,6 +206,10 @@ class AttnLib:
     def write_kv(self, args: PthAttnWriteArgs, stream: int | None = None) -> int:
         """The int8 cache writer (see include/pth_attn.h)."""
         return self.lib.pth_attn_write_kv(ctypes.byref(args), stream)
+
+    def last_kernel(self) -> str:
+        """Kernel of this thread's last attention launch (see the header)."""
+        return self.lib.pth_attn_last_kernel().decode()
 
     def last_error(self) -> str:
         return self.lib.pth_attn_last_error().decode()

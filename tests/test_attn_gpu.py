@@ -33,6 +33,11 @@ def _lib():
     return capi.AttnLib()
 
 
+def last_kernel() -> str:
+    """The kernel of this thread's last attention launch, by the C ABI or the op."""
+    return _lib().last_kernel()
+
+
 def _require_gpu():
     if not torch.cuda.is_available():
         pytest.fail("no GPU visible: the gpu tests need a gfx950 device")

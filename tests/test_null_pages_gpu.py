@@ -15,9 +15,11 @@ Here the same is done on every kernel family that can meet such a page:
 * per-wave staged (HND pages, windows > 4096 keys);
 * row-block (single split, 64-row tiles: windowed prefill chunks);
 * the any-block-size kernel (pages of 8 keys);
-* D = 64 and D = 256 (no windows there: the null pages are the block-table
-  tail past each request's last page, which the kernels address for the
-  16-key groups past a request's end).
+* wide-block (prefill with split partials, windowed at D = 128; one split at
+  D = 64 and 256);
+* D = 64 (page rows and per-wave staging) and D = 256 (no windows there: the
+  null pages are the block-table tail past each request's last page, which the
+  kernels address for the 16-key groups past a request's end).
 
 Every row-tile edge case is present: lengths that are not a multiple of 16 or
 32, so a chunk's second 16-key group lies past the end, and windows whose
@@ -32,6 +34,7 @@ import pytest
 import torch
 
 from cases import MAX_ABS, MEAN_ABS, Case, assert_parity, compare, materialize, oracle_of
+from test_attn_gpu import last_kernel
 
 pytestmark = pytest.mark.gpu
 
@@ -88,30 +91,42 @@ def run(b, *, num_splits: int, window: int, causal: bool) -> torch.Tensor:
     return out
 
 
-# (name, case kwargs, split counts). Block tables get 4 extra columns so that
-# every request has tail entries.
+# (name, case kwargs, split counts, kernel). Block tables get 4 extra columns so
+# that every request has tail entries.
 CASES = [
-    ("reg-cfg4", dict(q_lens=[16, 16, 16], seq_lens=[9000, 12345, 8203], window=2048), (0, 1, 7)),
+    ("reg-cfg4", dict(q_lens=[16, 16, 16], seq_lens=[9000, 12345, 8203], window=2048), (0, 1, 7),
+     None),  # one split: the row-block kernel
     ("reg-noncausal", dict(q_lens=[8, 8], seq_lens=[5003, 2100], window=2048, causal=False),
-     (0, 1)),
-    ("pagerows-q1", dict(q_lens=[1, 1, 1], seq_lens=[20000, 9001, 6007], window=5000), (0, 1)),
-    ("pagerows-q4", dict(q_lens=[4, 4], seq_lens=[30011, 12000], window=6000), (0, 3)),
+     (0, 1), "attn_fwd_paged_reg"),
+    ("pagerows-q1", dict(q_lens=[1, 1, 1], seq_lens=[20000, 9001, 6007], window=5000), (0, 1),
+     "attn_fwd_pagerows"),
+    ("pagerows-q4", dict(q_lens=[4, 4], seq_lens=[30011, 12000], window=6000), (0, 3),
+     "attn_fwd_pagerows"),
     ("staged-hnd", dict(q_lens=[1, 4], seq_lens=[15013, 9999], window=4500, layout="HND"),
-     (0, 1)),
+     (0, 1), "attn_fwd_staged"),
     ("staged-g8", dict(q_lens=[2, 1], seq_lens=[12007, 7005], Hq=32, Hkv=4, window=5000),
-     (0, 1)),
+     (0, 1), "attn_fwd_staged"),
     ("rows-prefill", dict(q_lens=[300, 77, 1], seq_lens=[4000, 3001, 2500], window=1000,
-                          is_prefill=True), (1,)),
+                          is_prefill=True), (1,), "attn_fwd_rows"),
+    ("wide-window", dict(q_lens=[700, 390], seq_lens=[4000, 3001], window=1000), (2, 5),
+     "attn_fwd_wide"),
+    ("wide-d64-tail", dict(q_lens=[400, 333], seq_lens=[1003, 1001], Hq=16, Hkv=4, D=64), (1, 3),
+     "attn_fwd_wide"),
+    ("wide-d256-tail", dict(q_lens=[600, 533], seq_lens=[1003, 1001], Hq=12, Hkv=2, D=256), (1, 3),
+     "attn_fwd_wide"),
     ("generic-bs8", dict(q_lens=[4, 1], seq_lens=[3001, 2003], window=700, block_size=8),
-     (0, 1)),
+     (0, 1), "attn_fwd_generic"),
     ("d256-tail", dict(q_lens=[4, 1, 1], seq_lens=[5003, 1001, 17], Hq=12, Hkv=2, D=256),
-     (0, 1)),
-    ("d64-tail", dict(q_lens=[4, 1], seq_lens=[3001, 33], Hq=16, Hkv=4, D=64), (0, 1)),
+     (0, 1), "attn_fwd_paged256"),
+    ("d64-tail", dict(q_lens=[4, 1], seq_lens=[3001, 33], Hq=16, Hkv=4, D=64), (0, 1),
+     "attn_fwd_staged64"),
+    ("d64-rows-tail", dict(q_lens=[4, 1, 1], seq_lens=[3001, 33, 1003], Hq=32, Hkv=8, D=64), (0, 1),
+     "attn_fwd_pagerows64"),
 ]
 
 
-@pytest.mark.parametrize("name,kw,splits", CASES, ids=[c[0] for c in CASES])
-def test_null_pages_are_never_used(name, kw, splits):
+@pytest.mark.parametrize("name,kw,splits,kernel", CASES, ids=[c[0] for c in CASES])
+def test_null_pages_are_never_used(name, kw, splits, kernel):
     if not torch.cuda.is_available():
         pytest.fail("no GPU visible")
     c = Case(name, seed=31, **kw)
@@ -127,6 +142,7 @@ def test_null_pages_are_never_used(name, kw, splits):
     for S in splits:
         S = c.plan().num_splits if S == 0 else S
         out = run(b, num_splits=S, window=c.window, causal=c.causal)
+        assert kernel is None or last_kernel() == kernel
         res = compare(out, None, ref_out, ref_lse, valid)
         print(f"  S={S} nulls={nulls} -> {res}", flush=True)
         assert_parity(res, name=f"null-{name}-S{S}", strict=False)

@@ -12,7 +12,7 @@ import pytest
 import torch
 
 from cases import Case, materialize
-from test_attn_gpu import check_case, run_op
+from test_attn_gpu import check_case, last_kernel, run_op
 
 pytestmark = pytest.mark.gpu
 
@@ -44,6 +44,12 @@ def cases():
 @pytest.mark.parametrize("case", list(cases()), ids=lambda c: c.name)
 def test_paged64(case, S):
     check_case(case, num_splits=S)
+    # Whole slot rows: NHD cells of 8 KV heads, at most 16 rows a tile.
+    rows = case.layout == "NHD" and case.Hkv == 8 and max(case.q_lens) * case.G <= 16
+    kernel = "attn_fwd_pagerows64" if rows else "attn_fwd_staged64"
+    if case.G == 64 and S == 1:  # a request's 64 rows reach the wide-block kernel's line
+        kernel = "attn_fwd_wide"
+    assert last_kernel() == kernel
 
 
 def test_paged64_repeats():
@@ -53,5 +59,6 @@ def test_paged64_repeats():
              D=64, seed=510)
     b = materialize(c, "cuda")
     first = run_op(b)
+    assert last_kernel() == "attn_fwd_pagerows64"
     for _ in range(5):
         assert torch.equal(run_op(b).view(torch.int16), first.view(torch.int16))

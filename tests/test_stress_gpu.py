@@ -1,8 +1,8 @@
 """Determinism under repetition: the same launch many times gives one result.
 
 The kernels hand data between waves through LDS (the page-row and staged
-kernels' shared chunk buffers, the row-block kernel's shared conversion and
-key-part merge, the combine's cross-wave merge) and between work-groups
+kernels' shared chunk buffers, the row-block and wide-block kernels' shared
+conversions, the key-part merge, the combines' cross-wave merges) and between work-groups
 through the workspace (split partials and the split-count marker that the
 combine reads). A missing barrier or wait shows up as an output that depends
 on timing. Each case below is launched LAUNCHES times through the C ABI into
@@ -24,27 +24,41 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda"
 LAUNCHES = 120
 
-# (case, forced num_splits or None for the planner's): one per kernel family.
+# (case, forced num_splits or None for the planner's, kernel): one per kernel family.
 STRESS = [
     (Case("pagerows-decode", q_lens=[1] * 64, seq_lens=uniform_lengths(64, 100, 6000, 90),
-          seed=90), None),
+          seed=90), None, "attn_fwd_pagerows"),
     (Case("pagerows-verify4", q_lens=[4] * 8, seq_lens=uniform_lengths(8, 100, 9000, 91),
-          seed=91), None),
-    (Case("staged-1kv", q_lens=[1], seq_lens=[3000], Hq=4, Hkv=1, seed=92), None),
+          seed=91), None, "attn_fwd_pagerows"),
+    (Case("staged-1kv", q_lens=[1], seq_lens=[3000], Hq=4, Hkv=1, seed=92), None,
+     "attn_fwd_staged"),
     (Case("regload-window", q_lens=[16] * 8, seq_lens=uniform_lengths(8, 600, 9000, 93),
-          window=512, seed=93), None),
+          window=512, seed=93), None, "attn_fwd_paged_reg"),
     (Case("rows-wide-and-parts", q_lens=[300, 1, 1, 40], seq_lens=[2000, 5000, 900, 700],
-          is_prefill=True, seed=94), 1),
+          is_prefill=True, seed=94), 1, "attn_fwd_rows"),
     (Case("paged256-decode", q_lens=[1, 1, 4], seq_lens=[8000, 300, 4000], Hq=12, Hkv=2, D=256,
-          seed=95), None),
+          seed=95), None, "attn_fwd_paged256"),
+    (Case("staged64", q_lens=[1, 2, 1], seq_lens=[3000, 700, 64], Hq=16, Hkv=4, D=64,
+          seed=96), None, "attn_fwd_staged64"),
     (Case("generic-d64", q_lens=[1, 2, 1], seq_lens=[3000, 700, 64], Hq=16, Hkv=4, D=64,
-          seed=96), None),
-    (Case("combine-many-splits", q_lens=[1], seq_lens=[40000], Hq=8, Hkv=2, seed=97), 300),
+          block_size=24, seed=96), None, "attn_fwd_generic"),
+    (Case("pagerows64", q_lens=[1, 4, 1, 2], seq_lens=[9000, 700, 64, 3333], Hq=32, Hkv=8, D=64,
+          seed=98), None, "attn_fwd_pagerows64"),
+    (Case("wide-split", q_lens=[700, 500, 40], seq_lens=[4000, 900, 3000], seed=99), 5,
+     "attn_fwd_wide"),
+    (Case("wide-d64", q_lens=[300, 1, 90], seq_lens=[2000, 1500, 90], Hq=16, Hkv=4, D=64,
+          seed=100), 1, "attn_fwd_wide"),
+    (Case("wide-d256", q_lens=[600, 700], seq_lens=[2500, 700], Hq=12, Hkv=2, D=256,
+          seed=101), 1, "attn_fwd_wide"),
+    (Case("combine-many-splits", q_lens=[1], seq_lens=[40000], Hq=8, Hkv=2, seed=97), 300,
+     "attn_fwd_staged"),
+    (Case("combine-rows", q_lens=[1] * 20, seq_lens=[300] * 7 + [40000] + [500] * 12, Hq=16,
+          Hkv=4, seed=102), 512, "attn_fwd_staged"),
 ]
 
 
-@pytest.mark.parametrize("case,S_force", STRESS, ids=[c.name for c, _ in STRESS])
-def test_repeated_launches_are_bitwise_identical(case, S_force):
+@pytest.mark.parametrize("case,S_force,kernel", STRESS, ids=[c.name for c, _, _ in STRESS])
+def test_repeated_launches_are_bitwise_identical(case, S_force, kernel):
     if not torch.cuda.is_available():
         pytest.fail("no GPU visible")
     from pth_flash_attn import capi
@@ -79,6 +93,7 @@ def test_repeated_launches_are_bitwise_identical(case, S_force):
         if i % 3 == 2:
             main.wait_stream(side)
         if first_out is None:
+            assert lib.last_kernel() == kernel
             torch.cuda.synchronize()
             assert not torch.isnan(out.float()).any(), "first launch left rows unwritten"
             first_out, first_lse = out.clone(), lse.clone()

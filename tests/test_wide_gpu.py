@@ -13,27 +13,20 @@ import numpy as np
 import pytest
 import torch
 
-from cases import (
-    Batch, Case, abs_v_batch, assert_parity, compare, materialize, oracle_of, tile_tokens,
-)
-from test_attn_gpu import check_case, run_capi, run_op
+from cases import Batch, Case, abs_v_batch, assert_parity, compare, materialize, oracle_of
+from test_attn_gpu import check_case, last_kernel, run_capi, run_op
 
 pytestmark = pytest.mark.gpu
 
 
+WIDE = "attn_fwd_wide"
+
+
 def min_rows(D: int, S: int) -> int:
-    """Mean query rows per request from which the launcher takes the kernel."""
+    """Mean query rows per request of the launcher's line (attn_launch.hip)."""
     if S == 1:
         return 384 if D == 256 else 64
     return 3072 if D == 256 else 1280
-
-
-def wide(c: Case, S: int) -> bool:
-    """The launcher's rule (attn_launch.hip)."""
-    plan = c.plan()
-    bq = tile_tokens(plan.wm, c.G, max(c.q_lens))
-    return (c.block_size % 16 == 0 and bq * c.G > 32 and (S > 1 or c.D != 128)
-            and c.T * c.G >= min_rows(c.D, S) * len(c.q_lens))
 
 
 def cases():
@@ -75,8 +68,8 @@ def cases():
 def test_wide(case, S):
     if S == 1 and case.D == 128:
         pytest.skip("the row-block kernel's launch")
-    assert wide(case, S), case.name
     check_case(case, num_splits=S)
+    assert last_kernel() == WIDE
 
 
 @pytest.mark.parametrize("D", [64, 128, 256])
@@ -84,9 +77,10 @@ def test_wide_op_and_repeats(D):
     """The op's launch (attention + combine) at the planner's split count, equal
     bit for bit over repeats."""
     c = Case(f"wide-op-d{D}", q_lens=[1000, 600], seq_lens=[2000, 633], Hq=8, Hkv=2, D=D, seed=430)
-    assert c.plan().num_splits > 1 and wide(c, c.plan().num_splits)
+    assert c.plan().num_splits > 1
     b = materialize(c, "cuda")
     first = run_op(b)
+    assert last_kernel() == WIDE
     ref, _, valid = oracle_of(b, threads=16)
     assert_parity(compare(first, None, ref, None, valid), name=c.name, strict=False)
     for _ in range(5):
@@ -102,7 +96,6 @@ def test_wide_large_v_scales(D, big):
     output: a term lies within 2^-17 = 7.6e-6 of itself, and the errors of a
     row's terms are as good as independent."""
     c = Case(f"wide-bigv-d{D}", q_lens=[800, 770], seq_lens=[800, 990], D=D, Hq=8, Hkv=2, seed=440)
-    assert wide(c, 3)
     b = materialize(c, "cuda")
     ch, bt = b.cache, b.cache.block_table.cpu()
     for r, (lo, hi, f) in enumerate([(100, 200, big), (400, 410, big * big)]):
@@ -111,6 +104,7 @@ def test_wide_large_v_scales(D, big):
     torch.cuda.synchronize()
     ref_out, ref_lse, valid = oracle_of(b)
     out, lse = run_capi(b, num_splits=3, out_dtype=torch.float32)
+    assert last_kernel() == WIDE
     o, r = out.cpu().numpy()[valid].astype(np.float64), ref_out[valid]
     assert np.isfinite(o).all()
     rel = np.abs(o - r) / np.abs(r).max(axis=-1, keepdims=True)
@@ -167,7 +161,6 @@ def _places(b, r, n):
 @pytest.mark.parametrize("D,S", [(64, 1), (64, 2), (128, 2), (256, 1), (256, 2)])
 def test_wide_small_weights(D, S, profile, x, ratio):
     c = _small_weight_case(D, S)
-    assert wide(c, S)
     b = materialize(c, "cuda")
     b.q.fill_(1.0)
     score, vs = profile(KEYS, 32 if D == 256 else 64, x, ratio)
@@ -183,6 +176,7 @@ def test_wide_small_weights(D, S, profile, x, ratio):
     ref_out, ref_lse, _ = oracle_of(lb, threads=16)
     abs_out, _, _ = oracle_of(abs_v_batch(lb), threads=16)
     out, lse = run_capi(b, num_splits=S, out_dtype=torch.float32)
+    assert last_kernel() == WIDE
     err = np.abs(out[-1:].cpu().numpy().astype(np.float64) - ref_out)
     worst = float((err / abs_out).max())
     print(f"d{D} S{S} {profile.__name__} x={x} ratio={ratio:.4f}: worst error / sum p|v| {worst:.3g}")
@@ -210,9 +204,9 @@ def test_wide_non_finite_scale(D, S, window, bad, stream):
     m = min_rows(D, 2) // 4
     c = Case(f"wide-nonfinite-d{D}", q_lens=[m + 70, m], seq_lens=[m + 300, m + 41], window=window, D=D,
              Hq=8, Hkv=2, seed=460)
-    assert wide(c, S)
     b = materialize(c, "cuda")
     clean, clean_lse = run_capi(b, num_splits=S, out_dtype=torch.float32)
+    assert last_kernel() == WIDE
     key = c.seq_lens[0] - c.q_lens[0] + 133  # within a block's tokens
     pages, slots = _places(b, 0, c.seq_lens[0])
     getattr(b.cache, stream)[pages[key], slots[key]] = bad
@@ -233,10 +227,10 @@ def test_wide_infinite_query(D, S):
     m = min_rows(D, 2) // 4
     c = Case(f"wide-infq-d{D}", q_lens=[m + 33], seq_lens=[m + 90], D=D, Hq=8, Hkv=2, q_dtype=torch.float16,
              seed=470)
-    assert wide(c, S)
     b = materialize(c, "cuda")
     b.cache.k_cache[..., 5] = -7
     clean, _ = run_capi(b, num_splits=S, out_dtype=torch.float32)
+    assert last_kernel() == WIDE
     row, head = 101, 3
     b.q[row, head, 5] = float("inf")
     out, _ = run_capi(b, num_splits=S, out_dtype=torch.float32)
