@@ -93,23 +93,39 @@ void set_cell_geometry(const PthAttnArgs& a, AttnParams& p) {
 // launches share at any R.
 constexpr int32_t kSharedCombineReqs = 16;
 
-// Query rows per request and KV head, on average, from which a launch runs on
-// the wide-block kernel: below, its few blocks of long steps leave the chip
-// idle. The keys of a request are not known here, so the line lies where the
-// shortest prefill (no prefix) is as fast on either side; a prefix only adds
-// to the gain. Measured with split partials, unit kernels -> wide, without a
-// prefix and with one of 3,000 keys: D = 128, 8 query heads per KV head, 160
-// tokens (1,280 rows) 33 -> 34 and 147 -> 82 us over 4 requests, 330 tokens 60
-// -> 55 and 288 -> 148; 4 query heads, 83 tokens 22 -> 27, 700 tokens 119 -> 91
-// and 599 -> 281. D = 64, 4 query heads, 160 tokens 31 -> 33 and 99 -> 71, 700
-// tokens 95 -> 85 and 375 -> 214. D = 256 (half the rows a block), 330 tokens 51
-// -> 56 and 213 -> 171, 700 tokens 94 -> 88 and 416 -> 307; one request of 700
-// 46 -> 49. On a single split there are blocks enough: D = 64, 64 requests of 24
-// tokens 30 -> 32 us, with 300 keys before them 76 -> 46; D = 256, 64 requests
-// of 83 tokens 42 -> 47 and 118 -> 101, 16 of 330 96 -> 79 and 168 -> 135.
-constexpr int64_t wide_min_rows(int32_t head_size, int32_t num_splits) {
-  if (num_splits == 1) return head_size == 256 ? 384 : 64;
-  return head_size == 256 ? 3072 : 1280;
+// Whether a prefill launch is faster on the wide-block kernel than on the unit
+// kernels, whose many small units fill the chip where its few blocks of long
+// steps do not. The host knows no lengths of keys, and a prefix always adds to the
+// gain, so the lines lie near where prefills without one are as fast on either
+// side on average (a block in use for one row of 256 costs what a full one does:
+// single sizes lie up to 11% to either side). At D = 64 on one split the line is
+// lower, since a prefix of 100 keys already gains several times what is lost
+// without. Batches of decodes and chunks in one launch gain at any mix (1.0 to 8.7
+// times). Measured, the tree before the kernel -> wide, us:
+//  * split partials, D = 128: no prefix, 8q / 1kv, one request of 164 tokens 16 ->
+//    20 us, of 480 28 -> 28, 4 of 164 18 -> 24, 4 of 336 32 -> 31; 16q / 4kv, one of
+//    327 23 -> 29, of 512 32 -> 32; 32q / 8kv, one of 327 31 -> 31, 4 of 400 61 -> 62,
+//    4 of 672 110 -> 89. Behind 1,000 keys the first of these still loses (25 ->
+//    31), 4 of 400 gain (158 -> 105). With few blocks in the launch more rows a
+//    request are needed: their product decides.
+//  * split partials, D = 64 (unit kernels there still on register loads): one
+//    request at one KV head 0.9 to 0.95 times, everything else 1.0 to 4 times.
+//    D = 256: 515 tokens (3,090 rows, half the rows a block) 46 -> 47, 4 of them 62
+//    -> 60, behind 1,000 keys 84 -> 71 and 124 -> 99.
+//  * one split, D = 64: 64 requests of 24 tokens 10.7 -> 12.2 (64q / 8kv, 16 of them
+//    7.6 -> 9.2), with 100 keys before them 39 -> 15 (16 -> 11), of 48 tokens 21 ->
+//    16 and 64 -> 25. D = 256: 64 requests of 65 tokens 26 -> 34, with 300 keys 80
+//    -> 68; of 83 39 -> 34 and 116 -> 70, of 100 45 -> 48 and 121 -> 95, of 150 78 ->
+//    68 and 176 -> 136; 16q / 4kv, 16 of 100 19 -> 20 and 41 -> 36; more heads per
+//    KV head do not help so few tokens (64q / 1kv, 64 of 40 tokens 51 -> 66).
+constexpr int64_t kWideRows = 1280, kWideRows256 = 3072;  // mean rows a request
+constexpr int64_t kWideWork = kWideRows * 8192;           // times rows of all heads
+bool wide_pays(const PthAttnArgs& a, int32_t group) {
+  const int64_t T = a.num_tokens, R = a.num_reqs, rows = T * group / R;
+  if (a.num_splits == 1)
+    return a.head_size == 64 ? rows >= 64 : rows >= 384 && T >= 80 * R;
+  if (a.head_size == 256) return rows >= kWideRows256;
+  return rows >= kWideRows && (a.head_size == 64 || T * a.num_q_heads >= kWideWork / rows);
 }
 
 }  // namespace
@@ -318,9 +334,7 @@ int32_t launch_attention(const PthAttnArgs& a, int32_t loader,
   // partials (their combine reads the split counts the kernel records, so
   // only on that path), and at the other head sizes.
   const bool wide = paged16 && !row_blocks && rows > 2 * kRowsPerWave &&
-                    (a.num_splits > 1 ? !fill_unused_splits : !d128) &&
-                    static_cast<int64_t>(a.num_tokens) * group >=
-                        a.num_reqs * wide_min_rows(a.head_size, a.num_splits);
+                    (a.num_splits > 1 ? !fill_unused_splits : !d128) && wide_pays(a, group);
   hipError_t err;
   if (wide) {
     p.blk_tok = wide_block_tokens(a.head_size, group);

@@ -25,8 +25,12 @@ WIDE = "attn_fwd_wide"
 def min_rows(D: int, S: int) -> int:
     """Mean query rows per request of the launcher's line (attn_launch.hip)."""
     if S == 1:
-        return 384 if D == 256 else 64
+        return 384 if D == 256 else 64  # at D = 256 of at least 80 tokens
     return 3072 if D == 256 else 1280
+
+
+# At D = 128 a launch needs 40 blocks of 256 rows as well at these lengths.
+HEADS = {D: {"Hq": 32 if D == 128 else 8, "Hkv": 8 if D == 128 else 2, "D": D} for D in (64, 128, 256)}
 
 
 def cases():
@@ -34,7 +38,7 @@ def cases():
         blk = 128 if D == 256 else 256  # rows of a block
         step = 32 if D == 256 else 64  # keys of a step
         m = min_rows(D, 2) // 4  # tokens of a request at four query heads per KV head
-        heads = {"Hq": 8, "Hkv": 2, "D": D}
+        heads = HEADS[D]
         # One block less, just, and more than full; keys at the step's edges.
         for i, (rows, keys) in enumerate([(blk - 4, 0), (blk, 1), (blk + 4, step - 1), (3 * blk, 17)]):
             q = m + rows // 4
@@ -49,13 +53,15 @@ def cases():
                    seed=412, Hq=12, Hkv=2, D=D)
         yield Case(f"wide-d{D}-bs528-pad", q_lens=[m + 70, m + 41], seq_lens=[m + 1200, m + 300],
                    block_size=528, pad_tokens=3, pad_page_bytes=72, seed=413, **heads)
-        yield Case(f"wide-d{D}-g64", q_lens=[m // 16 + 5, m // 16 + 3], seq_lens=[333, 90], Hq=64,
-                   Hkv=1, D=D, seed=414)
+        t = 78 if D == 256 else m // 16  # one split at D = 256: 80 tokens
+        yield Case(f"wide-d{D}-g64", q_lens=[t + 5, t + 3], seq_lens=[333, 90], Hq=64,
+                   Hkv=1, D=D, seed=414) if D != 128 else \
+            Case("wide-d128-g64", q_lens=[25, 23], seq_lens=[333, 90], Hq=192, Hkv=3, seed=414)
         yield Case(f"wide-d{D}-g1", q_lens=[4 * m + 300, 4 * m + 70], seq_lens=[4 * m + 300, 4 * m + 500],
-                   Hq=2, Hkv=2, D=D, seed=415)
+                   Hq=4 if D == 128 else 2, Hkv=4 if D == 128 else 2, D=D, seed=415)
         yield Case(f"wide-d{D}-many", q_lens=[m // 16 + i % 9 for i in range(70)],
                    seq_lens=[m // 16 + 9 + 3 * i for i in range(70)], seed=416, Hq=64, Hkv=1, D=D)
-    heads = {"Hq": 8, "Hkv": 2}
+    heads = HEADS[128]
     yield Case("wide-window", q_lens=[500, 400], seq_lens=[1200, 3000], window=64, seed=420, **heads)
     yield Case("wide-window-odd", q_lens=[531, 133], seq_lens=[2000, 800], window=333, seed=421, **heads)
     yield Case("wide-noncausal", q_lens=[600, 130], seq_lens=[900, 150], causal=False, seed=422, **heads)
@@ -68,6 +74,8 @@ def cases():
 def test_wide(case, S):
     if S == 1 and case.D == 128:
         pytest.skip("the row-block kernel's launch")
+    if S == 1 and case.D == 256 and case.T < 80 * len(case.q_lens):
+        pytest.skip("the unit kernels' launch")
     check_case(case, num_splits=S)
     assert last_kernel() == WIDE
 
@@ -146,8 +154,7 @@ def _tail(n, step, x, r):
 
 
 def _small_weight_case(D, S):
-    return Case(f"wide-small-d{D}", q_lens=[min_rows(D, 2) // 4 + 9], seq_lens=[KEYS], D=D, Hq=4, Hkv=1,
-                seed=450)
+    return Case(f"wide-small-d{D}", q_lens=[min_rows(D, 2) // 4 + 9], seq_lens=[KEYS], seed=450, **HEADS[D])
 
 
 def _places(b, r, n):
@@ -171,7 +178,7 @@ def test_wide_small_weights(D, S, profile, x, ratio):
     ch.v_scale[pages, slots] = torch.tensor(0.01 * vs, dtype=torch.float32, device="cuda")[:, None]
     torch.cuda.synchronize()
     # All rows have one query: the oracle on the last token's, which sees every key.
-    last = Case(c.name, q_lens=[1], seq_lens=[KEYS], D=D, Hq=4, Hkv=1)
+    last = Case(c.name, q_lens=[1], seq_lens=[KEYS], **HEADS[D])
     lb = Batch(last, ch, b.q[-1:], torch.tensor([0, 1], dtype=torch.int32, device="cuda"))
     ref_out, ref_lse, _ = oracle_of(lb, threads=16)
     abs_out, _, _ = oracle_of(abs_v_batch(lb), threads=16)
@@ -202,8 +209,8 @@ def test_wide_non_finite_scale(D, S, window, bad, stream):
     """A non-finite scale reaches the rows that see its key, and no other row of
     the block; a V scale never reaches a row's LSE."""
     m = min_rows(D, 2) // 4
-    c = Case(f"wide-nonfinite-d{D}", q_lens=[m + 70, m], seq_lens=[m + 300, m + 41], window=window, D=D,
-             Hq=8, Hkv=2, seed=460)
+    c = Case(f"wide-nonfinite-d{D}", q_lens=[m + 70, m], seq_lens=[m + 300, m + 41], window=window, seed=460,
+             **HEADS[D])
     b = materialize(c, "cuda")
     clean, clean_lse = run_capi(b, num_splits=S, out_dtype=torch.float32)
     assert last_kernel() == WIDE
@@ -223,17 +230,48 @@ def test_wide_non_finite_scale(D, S, window, bad, stream):
 @pytest.mark.parametrize("D,S", [(64, 1), (128, 2), (256, 1)])
 def test_wide_infinite_query(D, S):
     """A row whose fp16 query holds an infinity is NaN whatever the sign of the
-    keys' bytes there, and no other row changes."""
+    keys' bytes there (0 where it is split: a split without a sum is no split to
+    the combine), and no other row changes."""
     m = min_rows(D, 2) // 4
-    c = Case(f"wide-infq-d{D}", q_lens=[m + 33], seq_lens=[m + 90], D=D, Hq=8, Hkv=2, q_dtype=torch.float16,
-             seed=470)
+    c = Case(f"wide-infq-d{D}", q_lens=[m + 33] * 12, seq_lens=[m + 90] * 12, D=D, Hq=8, Hkv=2,
+             q_dtype=torch.float16, seed=470)
     b = materialize(c, "cuda")
     b.cache.k_cache[..., 5] = -7
     clean, _ = run_capi(b, num_splits=S, out_dtype=torch.float32)
     assert last_kernel() == WIDE
-    row, head = 101, 3
-    b.q[row, head, 5] = float("inf")
+    rows = torch.tensor([(m + 33) * r + 7 + 23 * r for r in range(12)], device="cuda")
+    heads = torch.arange(12, device="cuda") % 8
+    b.q[rows, heads, 5] = float("inf")
     out, _ = run_capi(b, num_splits=S, out_dtype=torch.float32)
-    assert torch.isnan(out[row, head]).all()
-    out[row, head] = clean[row, head]
+    bad = out[rows, heads]
+    nan = torch.isnan(bad).all(-1)
+    assert nan.any() if S > 1 else nan.all()
+    assert (nan | (bad == 0).all(-1)).all()
+    out[rows, heads] = clean[rows, heads]
     assert torch.equal(out.view(torch.int32), clean.view(torch.int32))
+
+
+@pytest.mark.parametrize("D,S,heads,q_lens,kernel", [
+    (64, 1, (8, 2), [16, 16], WIDE),
+    (64, 1, (8, 2), [16, 15], "attn_fwd_staged64"),
+    (256, 1, (12, 2), [80, 80], WIDE),
+    (256, 1, (12, 2), [80, 79], "attn_fwd_paged256"),
+    (256, 1, (8, 2), [96, 95], "attn_fwd_paged256"),
+    (256, 1, (64, 1), [79], "attn_fwd_paged256"),
+    (64, 4, (8, 1), [160], WIDE),
+    (64, 4, (8, 1), [159], "attn_fwd_staged64"),
+    (256, 4, (6, 1), [512], WIDE),
+    (256, 4, (6, 1), [511], "attn_fwd_paged256"),
+    (128, 4, (32, 4), [160, 160], WIDE),
+    (128, 4, (32, 4), [160, 159], "attn_fwd_staged"),
+    (128, 4, (32, 4), [202], "attn_fwd_staged"),  # 1,616 rows x 6,464 of all heads < 1,280 x 8,192
+    (128, 4, (32, 4), [203], WIDE),
+    (128, 4, (8, 1), [404], "attn_fwd_staged"),
+    (128, 4, (8, 1), [405], WIDE),
+])
+def test_launch_lines(D, S, heads, q_lens, kernel):
+    """Either side of the launcher's lines; the kernels agree at the parity gate."""
+    c = Case(f"line-d{D}", q_lens=q_lens, seq_lens=[q + 50 for q in q_lens], Hq=heads[0], Hkv=heads[1], D=D,
+             is_prefill=True, seed=480)
+    check_case(c, num_splits=S)
+    assert last_kernel() == kernel
