@@ -298,10 +298,13 @@ int32_t launch_attention(const PthAttnArgs& a, int32_t loader,
   const uint32_t cell = static_cast<uint32_t>(2 * a.head_size + 8);
   if (p.cell && a.head_size <= 128 && a.num_kv_heads == 8 && n_rg == 1 &&
       a.block_size % 16 == 0 && p.cell_head == cell && p.cell_slot == 8 * cell) {
-    bool inside = true;  // every stream of head h lies in bytes [cell h, cell h + cell) of the row
+    // Every stream of head h lies in bytes [cell h, cell h + cell) of the row, and
+    // one ends with the cell: whole rows are loaded, and streams that overlap
+    // (K as V) may leave the last cell's end outside the caller's memory.
+    uint32_t end = 0;
     for (int i = 0; i < 4; ++i)
-      inside = inside && p.cell_off[i] + (i < 2 ? static_cast<uint32_t>(a.head_size) : 4u) <= cell;
-    p.page_rows = inside ? 1 : 0;
+      end = std::max(end, p.cell_off[i] + (i < 2 ? static_cast<uint32_t>(a.head_size) : 4u));
+    p.page_rows = end == cell ? 1 : 0;
   }
 
   // Persistent grid. num_splits == 1: one wave per resident slot, but never

@@ -11,8 +11,8 @@ from __future__ import annotations
 import pytest
 import torch
 
-from cases import Case, materialize
-from test_attn_gpu import check_case, last_kernel, run_op
+from cases import Batch, Case, assert_parity, compare, materialize, oracle_of
+from test_attn_gpu import check_case, last_kernel, run_capi, run_op
 
 pytestmark = pytest.mark.gpu
 
@@ -62,3 +62,20 @@ def test_paged64_repeats():
     assert last_kernel() == "attn_fwd_pagerows64"
     for _ in range(5):
         assert torch.equal(run_op(b).view(torch.int16), first.view(torch.int16))
+
+
+@pytest.mark.parametrize("S", [1, 3])
+@pytest.mark.parametrize("D,kernel", [(64, "attn_fwd_staged64"), (128, "attn_fwd_staged")])
+def test_overlapping_streams(D, kernel, S):
+    """K as V in cells of the page-row size: no stream ends with the cell, so the
+    rest of the last one may be nobody's memory and whole rows are not loaded."""
+    c = Case(f"p64-k-as-v-d{D}", q_lens=[1, 2], seq_lens=[300, 77], Hq=32, Hkv=8, D=D, seed=511)
+    b = materialize(c, "cuda")
+    host = b.cache.to("cpu")
+    host.v_cache.copy_(host.k_cache)
+    host.v_scale.copy_(host.k_scale)
+    ref, ref_lse, valid = oracle_of(Batch(c, host, b.q.cpu(), b.qsl.cpu()))
+    b.cache.v_cache, b.cache.v_scale = b.cache.k_cache, b.cache.k_scale
+    out, lse = run_capi(b, num_splits=S)
+    assert last_kernel() == kernel
+    assert_parity(compare(out, lse, ref, ref_lse, valid), name=c.name, strict=False)
