@@ -48,17 +48,10 @@ constexpr float kNegInf = -__builtin_inff();
 template <int NC>
 constexpr int kBatch = 32 / NC;
 
-template <int kCtrl>
-__device__ __forceinline__ float dpp_f32(float v) {
-  return __builtin_bit_cast(float, dpp_i32<kCtrl>(__builtin_bit_cast(int, v)));
-}
-// Maximum over the 64 lanes (every lane; DPP within rows of 16 lanes, then
-// the four row maxima).
+// Maximum over the 64 lanes (every lane; within rows of 16 lanes, then the four
+// row maxima).
 __device__ __forceinline__ float wave_max(float x) {
-  x = fmaxf(x, dpp_f32<0xB1>(x));   // quad_perm [1, 0, 3, 2]
-  x = fmaxf(x, dpp_f32<0x4E>(x));   // quad_perm [2, 3, 0, 1]
-  x = fmaxf(x, dpp_f32<0x141>(x));  // row_half_mirror
-  x = fmaxf(x, dpp_f32<0x140>(x));  // row_mirror
+  x = lanes_max<16>(x);
   auto lane_f = [&](int l) {
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), l));
   };

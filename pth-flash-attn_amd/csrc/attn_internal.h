@@ -144,8 +144,8 @@ hipError_t launch_paged64_kernel(const AttnParams& p, dim3 grid, bool q_f16, hip
 hipError_t launch_rows_kernel(const AttnParams& p, dim3 grid, bool windowed, bool q_f16,
                               hipStream_t stream);
 int32_t rows_block_tokens(int32_t group);
-// The wide-block kernel (attn_wide.hip; paged cell caches, head size 64, 128
-// or 256, windowed / non-causal at 128 only, one split only at 64 and 256)
+// The wide-block kernel (attn_wide.hip; paged cell caches, split partials at
+// every head size, a single split at 64 and 256; windowed / non-causal at 128)
 // and the query tokens of one of its blocks.
 hipError_t launch_wide_kernel(const AttnParams& p, dim3 grid, bool windowed, bool q_f16,
                               int head_size, hipStream_t stream);

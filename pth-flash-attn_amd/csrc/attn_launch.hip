@@ -344,7 +344,8 @@ int32_t launch_attention(const PthAttnArgs& a, int32_t loader,
     const int64_t blocks =
         (static_cast<int64_t>(a.num_tokens) / p.blk_tok + a.num_reqs) * a.num_kv_heads;
     PA_REQUIRE(blocks < 0x7fffffff, "the block table exceeds 2^31 - 1 blocks");
-    const dim3 grid(static_cast<unsigned>(a.num_splits > 1 || blocks > wg_fill ? wg_fill : blocks));
+    const bool fill = a.num_splits > 1 || blocks > wg_fill;
+    const dim3 grid(static_cast<unsigned>(fill ? wg_fill : blocks));
     err = launch_wide_kernel(p, grid, windowed, a.q_dtype == PTH_ATTN_F16, a.head_size, stream);
   } else if (a.head_size == 64 && paged16) {
     const dim3 grid(static_cast<unsigned>(wg));

@@ -321,7 +321,8 @@ __device__ __forceinline__ void wave64_read(const char* slot, int h, int lane, C
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
     const int key = 32 * h + 16 * (e >> 2) + 4 * g + (e & 3);
-    ch.v[e] = *reinterpret_cast<const uint32_t*>(slot + kSlot64V + 64 * (key + (key >> 2)) + 4 * r16);
+    ch.v[e] =
+        *reinterpret_cast<const uint32_t*>(slot + kSlot64V + 64 * (key + (key >> 2)) + 4 * r16);
   }
   const int e = r16 & 7;
   ch.s = *reinterpret_cast<const float*>(slot + kSlot64S + (r16 < 8 ? 0 : 4 * kStep64) +
@@ -379,11 +380,15 @@ hipError_t launch_paged64_kernel(const AttnParams& p, dim3 grid, bool q_f16, hip
   const dim3 block(kFwdWaves * 64);
 #define PA_LAUNCH(K, St, F) hipLaunchKernelGGL((K<St, F>), grid, block, 0, stream, p)
   if (p.page_rows) {
-    if (st) { if (q_f16) PA_LAUNCH(attn_fwd_pagerows64, true, true); else PA_LAUNCH(attn_fwd_pagerows64, true, false); }
-    else { if (q_f16) PA_LAUNCH(attn_fwd_pagerows64, false, true); else PA_LAUNCH(attn_fwd_pagerows64, false, false); }
+    if (st && q_f16) PA_LAUNCH(attn_fwd_pagerows64, true, true);
+    else if (st) PA_LAUNCH(attn_fwd_pagerows64, true, false);
+    else if (q_f16) PA_LAUNCH(attn_fwd_pagerows64, false, true);
+    else PA_LAUNCH(attn_fwd_pagerows64, false, false);
   } else {
-    if (st) { if (q_f16) PA_LAUNCH(attn_fwd_staged64, true, true); else PA_LAUNCH(attn_fwd_staged64, true, false); }
-    else { if (q_f16) PA_LAUNCH(attn_fwd_staged64, false, true); else PA_LAUNCH(attn_fwd_staged64, false, false); }
+    if (st && q_f16) PA_LAUNCH(attn_fwd_staged64, true, true);
+    else if (st) PA_LAUNCH(attn_fwd_staged64, true, false);
+    else if (q_f16) PA_LAUNCH(attn_fwd_staged64, false, true);
+    else PA_LAUNCH(attn_fwd_staged64, false, false);
   }
 #undef PA_LAUNCH
   return hipGetLastError();

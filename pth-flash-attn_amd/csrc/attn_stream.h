@@ -74,6 +74,22 @@ __device__ __forceinline__ int dpp_i32(int v) {
   return __builtin_amdgcn_update_dpp(0, v, kCtrl, kRowMask, 0xf, true);
 }
 
+template <int kCtrl>
+__device__ __forceinline__ float dpp_f32(float v) {
+  return __builtin_bit_cast(float, dpp_i32<kCtrl>(__builtin_bit_cast(int, v)));
+}
+
+// Maximum over each kLanes (8, 16, 32) consecutive lanes, in every one of them.
+template <int kLanes>
+__device__ __forceinline__ float lanes_max(float x) {
+  x = fmaxf(x, dpp_f32<0xB1>(x));   // quad_perm [1, 0, 3, 2]
+  x = fmaxf(x, dpp_f32<0x4E>(x));   // quad_perm [2, 3, 0, 1]
+  x = fmaxf(x, dpp_f32<0x141>(x));  // row_half_mirror
+  if constexpr (kLanes > 8) x = fmaxf(x, dpp_f32<0x140>(x));  // row_mirror
+  if constexpr (kLanes > 16) x = fmaxf(x, __shfl_xor(x, 16));
+  return x;
+}
+
 // Inclusive prefix sum over the 64 lanes: within each row of 16 lanes by
 // row shifts of 1, 2, 4 and 8 (lanes shifted in from outside the row add 0),
 // then lane 15's running total into rows 1 and 3 and lane 31's into rows 2

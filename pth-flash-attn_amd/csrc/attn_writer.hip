@@ -24,7 +24,7 @@
 #include <cmath>
 #include <string>
 
-#include "attn_internal.h"
+#include "attn_stream.h"
 
 namespace pa {
 namespace {
@@ -85,23 +85,6 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef u32x2 u32x2_a4 __attribute__((aligned(4)));
 
-template <int kCtrl>
-__device__ __forceinline__ float dpp_max(float x) {
-  return fmaxf(x, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(
-                                                0, __builtin_bit_cast(int, x), kCtrl, 0xf, 0xf, true)));
-}
-
-// Maximum over the kLanes (8, 16, 32) consecutive lanes that share a row.
-template <int kLanes>
-__device__ __forceinline__ float lanes_max(float x) {
-  x = dpp_max<0xB1>(x);   // quad_perm [1, 0, 3, 2]
-  x = dpp_max<0x4E>(x);   // quad_perm [2, 3, 0, 1]
-  x = dpp_max<0x141>(x);  // row_half_mirror
-  if constexpr (kLanes > 8) x = dpp_max<0x140>(x);  // row_mirror
-  if constexpr (kLanes > 16) x = fmaxf(x, __shfl_xor(x, 16));
-  return x;
-}
-
 // Eight consecutive elements of a row.
 template <int kType>
 struct Eight {
@@ -112,11 +95,12 @@ struct Eight {
   }
   __device__ __forceinline__ float at(int i) const {
     if constexpr (kType == PTH_ATTN_F32) {
-      const uint32_t x = w[i >> 2][i & 3];  // a value: a bit cast of the element itself reads element 0
+      const uint32_t x = w[i >> 2][i & 3];  // a value: a cast of the element reads element 0
       return __builtin_bit_cast(float, x);
     } else {
       const uint16_t h = static_cast<uint16_t>(w[0][i >> 1] >> (16 * (i & 1)));
-      if constexpr (kType == PTH_ATTN_F16) return static_cast<float>(__builtin_bit_cast(_Float16, h));
+      if constexpr (kType == PTH_ATTN_F16)
+        return static_cast<float>(__builtin_bit_cast(_Float16, h));
       else return static_cast<float>(__builtin_bit_cast(__bf16, h));
     }
   }
@@ -158,7 +142,8 @@ __global__ __launch_bounds__(256) void write_kv_int8_wide(const WriteParams w) {
   constexpr int kElt = kType == PTH_ATTN_F32 ? 4 : 2;
   const uint32_t item = blockIdx.x * (256u / kLanes) + threadIdx.x / kLanes;
   const int l = threadIdx.x % kLanes;
-  const uint32_t items = static_cast<uint32_t>(w.num_tokens) * static_cast<uint32_t>(w.num_kv_heads);
+  const uint32_t items =
+      static_cast<uint32_t>(w.num_tokens) * static_cast<uint32_t>(w.num_kv_heads);
   if (item >= items) return;  // a row's lanes together
   const uint32_t tok = w.heads_div.div(item);
   const uint32_t head = item - tok * static_cast<uint32_t>(w.num_kv_heads);
@@ -176,8 +161,10 @@ __global__ __launch_bounds__(256) void write_kv_int8_wide(const WriteParams w) {
     return const_cast<char*>(s.base) + static_cast<int64_t>(page) * s.s_block +
            static_cast<int64_t>(in_page) * s.s_slot + static_cast<int64_t>(head) * s.s_head;
   };
-  quantize_eight<kLanes, kType>(k, cell(w.k) + 8 * l, reinterpret_cast<float*>(cell(w.ks)), l == 0, live);
-  quantize_eight<kLanes, kType>(v, cell(w.v) + 8 * l, reinterpret_cast<float*>(cell(w.vs)), l == 0, live);
+  quantize_eight<kLanes, kType>(k, cell(w.k) + 8 * l, reinterpret_cast<float*>(cell(w.ks)),
+                                l == 0, live);
+  quantize_eight<kLanes, kType>(v, cell(w.v) + 8 * l, reinterpret_cast<float*>(cell(w.vs)),
+                                l == 0, live);
 }
 
 template <int D>
@@ -273,8 +260,9 @@ int32_t launch_write_kv(const PthAttnWriteArgs& a, hipStream_t stream) {
     return reinterpret_cast<uintptr_t>(s.base) % 4 == 0 && s.s_block % 4 == 0 &&
            s.s_slot % 4 == 0 && s.s_head % 4 == 0;
   };
-  const bool wide = rows16(w.key, w.s_k_tok, w.s_k_head) && rows16(w.value, w.s_v_tok, w.s_v_head) &&
-                    cells4(w.k) && cells4(w.v) && items < 0x7fffffff && w.num_slots < 0x7fffffff;
+  const bool wide = rows16(w.key, w.s_k_tok, w.s_k_head) &&
+                    rows16(w.value, w.s_v_tok, w.s_v_head) && cells4(w.k) && cells4(w.v) &&
+                    items < 0x7fffffff && w.num_slots < 0x7fffffff;
   if (wide) {
     w.bs_div = Div32::make(static_cast<uint32_t>(a.block_size));
     w.heads_div = Div32::make(static_cast<uint32_t>(a.num_kv_heads));

@@ -35,8 +35,8 @@ def test_long_row_among_short_ones(D, chunks):
     this small is a split) beside rows of two, on the kernel that cuts a long
     row into runs: one block, the last wave's run short or empty, runs of more
     than a block; output and LSE."""
-    c = Case(f"combine-row-d{D}-{chunks}", q_lens=[1] * 17, seq_lens=[40] * 8 + [32 * chunks - 5] + [60] * 8,
-             Hq=4, Hkv=1, D=D, seed=620)
+    c = Case(f"combine-row-d{D}-{chunks}", q_lens=[1] * 17,
+             seq_lens=[40] * 8 + [32 * chunks - 5] + [60] * 8, Hq=4, Hkv=1, D=D, seed=620)
     assert c.plan().num_splits > chunks
     b = materialize(c, "cuda")
     ref, ref_lse, valid = oracle_of(b, threads=16)

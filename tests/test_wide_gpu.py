@@ -30,7 +30,8 @@ def min_rows(D: int, S: int) -> int:
 
 
 # At D = 128 a launch needs 40 blocks of 256 rows as well at these lengths.
-HEADS = {D: {"Hq": 32 if D == 128 else 8, "Hkv": 8 if D == 128 else 2, "D": D} for D in (64, 128, 256)}
+HEADS = {64: {"Hq": 8, "Hkv": 2, "D": 64}, 128: {"Hq": 32, "Hkv": 8, "D": 128},
+         256: {"Hq": 8, "Hkv": 2, "D": 256}}
 
 
 def cases():
@@ -154,7 +155,8 @@ def _tail(n, step, x, r):
 
 
 def _small_weight_case(D, S):
-    return Case(f"wide-small-d{D}", q_lens=[min_rows(D, 2) // 4 + 9], seq_lens=[KEYS], seed=450, **HEADS[D])
+    return Case(f"wide-small-d{D}", q_lens=[min_rows(D, 2) // 4 + 9], seq_lens=[KEYS], seed=450,
+                **HEADS[D])
 
 
 def _places(b, r, n):
@@ -174,8 +176,9 @@ def test_wide_small_weights(D, S, profile, x, ratio):
     pages, slots = _places(b, 0, KEYS)
     ch = b.cache
     ch.k_cache[pages, slots] = 1  # score = sqrt(D) k_scale
-    ch.k_scale[pages, slots] = torch.tensor(score * np.log(2) / np.sqrt(D), dtype=torch.float32, device="cuda")[:, None]
-    ch.v_scale[pages, slots] = torch.tensor(0.01 * vs, dtype=torch.float32, device="cuda")[:, None]
+    f32 = {"dtype": torch.float32, "device": "cuda"}
+    ch.k_scale[pages, slots] = torch.tensor(score * np.log(2) / np.sqrt(D), **f32)[:, None]
+    ch.v_scale[pages, slots] = torch.tensor(0.01 * vs, **f32)[:, None]
     torch.cuda.synchronize()
     # All rows have one query: the oracle on the last token's, which sees every key.
     last = Case(c.name, q_lens=[1], seq_lens=[KEYS], **HEADS[D])
@@ -209,8 +212,8 @@ def test_wide_non_finite_scale(D, S, window, bad, stream):
     """A non-finite scale reaches the rows that see its key, and no other row of
     the block; a V scale never reaches a row's LSE."""
     m = min_rows(D, 2) // 4
-    c = Case(f"wide-nonfinite-d{D}", q_lens=[m + 70, m], seq_lens=[m + 300, m + 41], window=window, seed=460,
-             **HEADS[D])
+    c = Case(f"wide-nonfinite-d{D}", q_lens=[m + 70, m], seq_lens=[m + 300, m + 41],
+             window=window, seed=460, **HEADS[D])
     b = materialize(c, "cuda")
     clean, clean_lse = run_capi(b, num_splits=S, out_dtype=torch.float32)
     assert last_kernel() == WIDE
@@ -271,7 +274,7 @@ def test_wide_infinite_query(D, S):
 ])
 def test_launch_lines(D, S, heads, q_lens, kernel):
     """Either side of the launcher's lines; the kernels agree at the parity gate."""
-    c = Case(f"line-d{D}", q_lens=q_lens, seq_lens=[q + 50 for q in q_lens], Hq=heads[0], Hkv=heads[1], D=D,
-             is_prefill=True, seed=480)
+    c = Case(f"line-d{D}", q_lens=q_lens, seq_lens=[q + 50 for q in q_lens], Hq=heads[0],
+             Hkv=heads[1], D=D, is_prefill=True, seed=480)
     check_case(c, num_splits=S)
     assert last_kernel() == kernel
